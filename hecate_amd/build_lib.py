@@ -12,7 +12,8 @@ ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libhecate_moe.so")
-SOURCES = ["common.hip", "decode.hip", "router.hip", "norm.hip", "prefill.hip", "cputier_gpu.hip", "shared_gemm.hip"]
+SOURCES = ["common.hip", "decode.hip", "router.hip", "norm.hip", "prefill.hip", "pgemm_gu.hip", "pgemm_dn.hip",
+           "cputier_gpu.hip", "shared_gemm.hip"]
 HOST_SOURCES = ["cputier.cpp"]                 # host-only C++ (the CPU expert tier), built with the host compiler
 CXX = os.environ.get("CXX_HOST", "g++")
 # AVX2 / FMA / F16C is the x86-64-v3 level (every AVX2 EPYC and Xeon); no fp contraction, so the q8_0 arithmetic
@@ -58,7 +59,7 @@ def _compile_host(src):
 
 def build(verbose=False):
     os.makedirs(OBJ, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=min(4, len(SOURCES) + len(HOST_SOURCES))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(SOURCES) + len(HOST_SOURCES))) as ex:
         jobs = [ex.submit(_compile, s) for s in SOURCES] + [ex.submit(_compile_host, s) for s in HOST_SOURCES]
         results = [j.result() for j in jobs]
     for _, err in results:

@@ -3,16 +3,15 @@
 //
 // Dispatch: picks sorted by (expert, flat index) by a counting sort with per-block histograms and in-block ranks, so
 // the order equals a stable argsort of the selection; row blocks {expert, first pick, picks, 0} of at most bm picks.
-// GEMMs: workgroup = (row block of <= 128 picks of one expert, 128 gate/up or 256 down output columns); see
-// pgemm_kernel. gu fuses act = silu(g) * u * w (f16), down writes d = W_d act (fp32), fin adds each
+// GEMMs: workgroup = (row block of picks of one expert, 128 gate/up or 256 down output columns); see pgemm.h, and
+// pgemm16_kernel for the long prefill. gu fuses act = silu(g) * u * w (f16), down writes d = W_d act (fp32), fin adds each
 // token's picks into out in top-k order (or with atomics, as p4_fin_kernel, when no inverse map is given). The shared
 // expert's projections run on the dense MFMA GEMMs of shared_gemm.hip.
-#include "hmoe_dev.h"
+#include "pgemm.h"
 
 namespace hmoe {
 
-constexpr int PB = 128;                     // picks per row block (dispatch bm <= 128)
-constexpr int PT = 256;                     // threads
+constexpr int PB = PG_PB;                   // picks per row block half (dispatch bm <= 2 PB)
 constexpr int DBLK = 256;                   // picks per dispatch block
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -131,44 +130,17 @@ __global__ void __launch_bounds__(DBLK) disp_place_kernel(const int64_t* __restr
 // ---------------------------------------------------------------------------------------------------------------
 // grouped GEMMs
 // ---------------------------------------------------------------------------------------------------------------
-struct Block { int e, p0, rows; };
-
-// The workgroup's row block and column block. The dispatcher deals a launch's workgroups round-robin over the 8
-// XCDs (workgroup i runs on XCD i % 8), each with its own L2: the column blocks of one row block go to consecutive
-// workgroups of one XCD, so they run together and read the block's input rows from that XCD's L2 (one fetch from
-// memory instead of one per column block). The grid's x extent is a multiple of 8 (pgemm_grid).
-// (the grid's extents come from the launch's own arguments: gridDim reads the dispatch packet, a round trip to the
-// queue's memory at every workgroup start)
-__device__ __forceinline__ void xcd_tile(int& rb, int& cb, int gx, int ny)
-{
-    const int i = blockIdx.x + gx * blockIdx.y, j = i >> 3;
-    rb = (j / ny) * 8 + (i & 7);
-    cb = j % ny;
-}
-
-static dim3 pgemm_grid(int nrb, int ny) { return dim3((nrb + 7) & ~7, ny); }
-
-// row block rb of the plan: up to 2 PB picks (the dispatch's bm <= 256), run as halves of <= PB picks; a block
-// whose expert or picks fall outside the tables (np picks) is skipped, so a caller's malformed plan reads nothing
-// out of bounds
-__device__ __forceinline__ bool get_block(const int* rbt, int nrb, const int* meta, int n_tab, int np, int rb, Block& b)
-{
-    if (rb >= nrb || (meta && rb >= meta[1])) return false;
-    b.e = rbt[4 * rb]; b.p0 = rbt[4 * rb + 1]; b.rows = min(rbt[4 * rb + 2], 2 * PB);
-    return b.e >= 0 && b.e < n_tab && b.rows > 0 && b.p0 >= 0 && b.p0 <= np - b.rows;
-}
-
-// A pipelined grouped GEMM for both projections. Workgroup = (row block of <= 128 picks of one expert, 64 NS output
-// columns); wave w of column block cb owns output strips nb0 = NWV NS cb + NS w .. + NS (16 rows each) of NMAT
-// matrices (gate and up: NS = 2, or down: NS = 4), so every wave holds 4 weight fragments per k step and reads each
-// 16-pick input fragment from LDS once for 4 MFMAs. Per 128-k group kg:
+// The long prefill's grouped GEMM for both projections (blocks of up to 256 picks in one pass; the other chunks run on
+// pgemm.h's). Workgroup = (row block of <= 256 picks of one expert, 64 NS output columns), 8 waves; wave w of column block
+// cb owns output strips nb0 = NWV NS cb + NS w .. + NS (16 rows each) of NMAT matrices (gate and up: NS = 1, down: NS = 2),
+// so every dequantised fragment feeds up to 16 pick tiles. Per 128-k group kg:
 //   * the block's input rows are staged in LDS as f16 by direct global-to-LDS loads (double-buffered, one barrier
 //     per group): the next group's rows load while this group computes;
 //   * the weight tiles come from a ring of D groups of unconditional 16-byte loads, issued D - 1 groups ahead, so HBM
 //     latency hides behind that many groups of MFMA work; each tile is loaded once per workgroup; the lane's row
 //     scales come 4 groups at a time (one 8-byte load per fragment every fourth group);
-//   * each k step dequantises the 4 weight fragments (exact f16 codes times the f16 group scale) and runs the
-//     16x16x32 MFMA against the block's 16-pick tiles (up to 8).
+//   * each k step dequantises the weight fragments (exact f16 codes times the f16 group scale) and runs the
+//     16x16x32 MFMA against the block's 16-pick tiles.
 // Every vector-memory instruction costs issue time on the SIMD beside the MFMA and dequantisation work, so the loads
 // are few and their addresses cheap: uniform bases in scalar registers with 32-bit lane offsets.
 template <int NMAT, int NS>
@@ -177,15 +149,9 @@ struct PFetch
     u32x4 q[NS][NMAT];
 };
 
-// epilogues: gate/up -> act f16 (EPI_ACT) or the raw gate and up sums (EPI_RAW, fp32 [2][ps][I], the test entry of
-// moe4t); down -> d f16 rows for the ordered combine (EPI_D16), d fp32 rows (EPI_D, the moe4t.gemm test entry) or
-// added into out[tok] with fp32 atomics (EPI_FIN, moe4t.cu's down epilogue)
-enum { EPI_ACT = 0, EPI_RAW = 1, EPI_D = 2, EPI_FIN = 3, EPI_D16 = 4 };
-
-// NTT: 16-pick tiles per pass (8: 128 picks, 4 waves; 16: 256 picks, 8 waves, one pass for the long prefill's 256-pick
-// blocks, each dequantised weight fragment feeding twice the MFMAs); NWV waves, each staging two tiles
-template <int NMAT, int NS, int D, int EPI = NMAT == 2 ? EPI_ACT : EPI_D, int NTT = 8, int NWV = 4>
-__global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2))) pgemm_kernel(
+// NTT: 16-pick tiles per pass; NWV waves, each staging two tiles
+template <int NMAT, int NS, int D, int EPI, int NTT = 16, int NWV = 8>
+__global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2))) pgemm16_kernel(
     const _Float16* __restrict__ xin, const int* __restrict__ tok, const float* __restrict__ wt,
     const int* __restrict__ rbt, int nrb, const int* __restrict__ meta, int n_tab,
     const int64_t* __restrict__ w0, const int64_t* __restrict__ w1, const int64_t* __restrict__ s0,
@@ -608,18 +574,18 @@ static int moe4p_run(const void* x, const int* tok, const float* wt, const int* 
         xb = (const uint16_t*) gu;
     }
     _Float16* a = (_Float16*) ar;
-    // gate/up: 64 x 2 output columns per workgroup (NS 2); down: 64 x 4 (NS 4), into d rows for the ordered combine
-    // (inv given) or added into out[tok] by its epilogue (no inverse map: the atomic combine of p4_fin_kernel)
+    // gate/up, then down into d rows for the ordered combine (inv given) or added into out[tok] by its epilogue (no
+    // inverse map: the atomic combine of p4_fin_kernel)
     if (nrb > 0)
     {
-        pgemm_kernel<2, 2, 2><<<pgemm_grid(nrb, I / 128), PT, 0, st>>>((const _Float16*) xb, tok, wt, rbt, nrb, meta,
-            n_tab, gw, uw, gs, us, a, nullptr, T, 0, npos);
-        if (inv)
-            pgemm_kernel<1, 4, 2, EPI_D16><<<pgemm_grid(nrb, H / 256), PT, 0, st>>>(a, nullptr, nullptr, rbt, nrb, meta,
-                n_tab, dw, nullptr, ds, nullptr, nullptr, d, T, 0, npos);
-        else
-            pgemm_kernel<1, 4, 2, EPI_FIN><<<pgemm_grid(nrb, H / 256), PT, 0, st>>>(a, tok, nullptr, rbt, nrb, meta, n_tab,
-                dw, nullptr, ds, nullptr, nullptr, nullptr, T, 0, npos, out);
+        PgArgs g{};
+        g.xin = (const _Float16*) xb; g.tok = tok; g.wt = wt; g.rbt = rbt; g.meta = meta;
+        g.w0 = gw; g.w1 = uw; g.s0 = gs; g.s1 = us; g.out = a;
+        g.nrb = nrb; g.n_tab = n_tab; g.T = T; g.np = npos; g.ps = ps;
+        if (int rc = grouped_gate_up(g, EPI_ACT, st)) return rc;
+        g.xin = a; g.w0 = dw; g.s0 = ds; g.w1 = g.s1 = nullptr;
+        g.out = inv ? d : out;
+        if (int rc = grouped_down(g, inv ? EPI_D16 : EPI_FIN, st)) return rc;
     }
     const bool sh = sh_gw != nullptr;
     if (sh)
@@ -748,14 +714,14 @@ static int moe4t_run(const void* x, const int* tok, const float* wt, const int* 
     {
         // 256-pick blocks in one pass: 8 waves, each one 16-row strip of gate and of up (or two of down) against the
         // block's 16 pick tiles
-        pgemm_kernel<2, 1, 4, EPI_ACT, 16, 8><<<pgemm_grid(nrb, I / 128), 512, 0, st>>>(xh, tok, wt, rbt, nrb, meta, n_tab,
+        pgemm16_kernel<2, 1, 4, EPI_ACT><<<pgemm_grid(nrb, I / 128), 512, 0, st>>>(xh, tok, wt, rbt, nrb, meta, n_tab,
             gw, uw, gs, us, (_Float16*) ar, nullptr, T, 0, npos);
         // (d held the f16 copy of x, which the gate/up GEMM has consumed by now: the down rows may overwrite it)
         if (inv)
-            pgemm_kernel<1, 2, 4, EPI_D16, 16, 8><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar,
+            pgemm16_kernel<1, 2, 4, EPI_D16><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar,
                 nullptr, nullptr, rbt, nrb, meta, n_tab, dw, nullptr, ds, nullptr, nullptr, d, T, 0, npos);
         else
-            pgemm_kernel<1, 2, 4, EPI_FIN, 16, 8><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar, tok,
+            pgemm16_kernel<1, 2, 4, EPI_FIN><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar, tok,
                 nullptr, rbt, nrb, meta, n_tab, dw, nullptr, ds, nullptr, nullptr, nullptr, T, 0, npos, out);
     }
     if (inv && ob) pfin_kernel<PF_FIN><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, -1, out, ob);
@@ -801,11 +767,8 @@ extern "C" int hmoe_moe4t_gemm(const void* xs, int rows, const int* rbt, int nrb
     HMOE_REQUIRE(((uintptr_t) xs & 15) == 0 && ((uintptr_t) out & 15) == 0, "moe4t_gemm: alignment");
     if (nrb == 0) return HMOE_OK;
     hipStream_t st = (hipStream_t) stream;
-    if (down)
-        pgemm_kernel<1, 4, 2><<<pgemm_grid(nrb, H / 256), PT, 0, st>>>((const _Float16*) xs, nullptr, nullptr, rbt, nrb,
-            nullptr, n_tab, w0, nullptr, s0, nullptr, nullptr, out, rows, 0, rows);
-    else
-        pgemm_kernel<2, 2, 2, EPI_RAW><<<pgemm_grid(nrb, I / 128), PT, 0, st>>>((const _Float16*) xs, nullptr, nullptr,
-            rbt, nrb, nullptr, n_tab, w0, w1, s0, s1, nullptr, out, rows, 0, rows, nullptr, ps);
-    return HMOE_LAUNCHED("moe4t_gemm");
+    PgArgs g{};
+    g.xin = (const _Float16*) xs; g.rbt = rbt; g.w0 = w0; g.w1 = w1; g.s0 = s0; g.s1 = s1; g.out = out;
+    g.nrb = nrb; g.n_tab = n_tab; g.T = rows; g.np = rows; g.ps = ps;
+    return down ? grouped_down(g, EPI_D, st) : grouped_gate_up(g, EPI_RAW, st);
 }
