@@ -40,17 +40,17 @@ struct Block { int e, p0, rows; };
 // The workgroup's row block and column block. The dispatcher deals a launch's workgroups round-robin over the 8
 // XCDs (workgroup i runs on XCD i % 8), each with its own L2: the column blocks of one row block go to consecutive
 // workgroups of one XCD, so they run together and read the block's input rows from that XCD's L2 (one fetch from
-// memory instead of one per column block). The grid's x extent is a multiple of 8 (pgemm_grid).
-// (the grid's extents come from the launch's own arguments: gridDim reads the dispatch packet, a round trip to the
-// queue's memory at every workgroup start)
-__device__ __forceinline__ void xcd_tile(int& rb, int& cb, int gx, int ny)
+// memory instead of one per column block). i: the workgroup's index among nrb (rounded up to 8) x ny.
+// (the extents come from the launch's own arguments: gridDim reads the dispatch packet, a round trip to the queue's
+// memory at every workgroup start)
+__device__ __forceinline__ void xcd_tile(int i, int& rb, int& cb, int ny)
 {
-    const int i = blockIdx.x + gx * blockIdx.y, j = i >> 3;
+    const int j = i >> 3;
     rb = (j / ny) * 8 + (i & 7);
     cb = j % ny;
 }
 
-inline dim3 pgemm_grid(int nrb, int ny) { return dim3((nrb + 7) & ~7, ny); }
+inline dim3 pgemm_grid(int nrb, int ny) { return dim3(((nrb + 7) & ~7) * ny); }
 
 // a scalar load from memory that no kernel of the launch writes: under the weight stream a vector load returns behind
 // every load the CU has in flight (over 1 us), a scalar load does not wait for them. The address must be the same in
@@ -89,7 +89,18 @@ struct PgArgs
     void* out;
     int nrb, n_tab, T, np, ps;
     int ncb;                                // column blocks per workgroup (set by the launchers)
+    // the shared expert (row-major f16 [N][K], NULL: none) on every one of the T tokens in the same launch: its rows follow
+    // the picks' (row ps + t of the act, and of down's rows)
+    const _Float16* sh0;
+    const _Float16* sh1;
+    int nsh, sh_rows;                       // its token blocks and the tokens of each (set by the launchers)
 };
+// the shared expert's token blocks: of equal size, whole tiles, at most PG_PB
+inline void pg_shared_blocks(PgArgs& a)
+{
+    a.nsh = a.sh0 ? (a.T + PG_PB - 1) / PG_PB : 0;
+    a.sh_rows = a.nsh ? (((a.T + a.nsh - 1) / a.nsh) + 15) & ~15 : 0;
+}
 int grouped_gate_up(const PgArgs& a, int epi, hipStream_t st);
 int grouped_down(const PgArgs& a, int epi, hipStream_t st);
 
@@ -98,9 +109,18 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t pg_rsrc(uint64_t p, uint32_t b
     return __builtin_amdgcn_make_buffer_rsrc((void*) p, (short) 0, (int) bytes, 0x00020000);
 }
 
-// the epilogue of one tile: lane holds output rows n .. n + 4 of pick pk (row p0 + pk)
-template <int EPI, int NT>
-__device__ __forceinline__ void pg_store(const PgArgs& a, const Block& b, int nb0, int lane, const f32x4 (&acc)[4][NT])
+// 16 bytes per lane from a buffer to LDS (lane l at lds + 16 l). (Device pass only: the host target knows no 16-byte form.)
+__device__ __forceinline__ void pg_load_lds(__amdgpu_buffer_rsrc_t rs, u32x4* lds, uint32_t voff, int soff)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*) lds, 16, (int) voff, soff, 0, 0);
+#endif
+}
+
+// the epilogue of a pass: lane holds output rows n .. n + 4 of pick pk (row p0 + pk of the output). SH: the shared expert's
+// (weight 1)
+template <int EPI, int NT, bool SH>
+__device__ __forceinline__ void pg_store(const PgArgs& a, int p0, int rows, int nb0, int lane, const f32x4 (&acc)[4][NT])
 {
     constexpr int NMAT = EPI == EPI_ACT || EPI == EPI_RAW ? 2 : 1, NS = 4 / NMAT, NOUT = NMAT == 2 ? I : H;
     // (an opaque copy of the lane: no address formed here is kept in registers across the k loop)
@@ -110,9 +130,9 @@ __device__ __forceinline__ void pg_store(const PgArgs& a, const Block& b, int nb
     for (int tt = 0; tt < NT; ++tt)
     {
         const int pk = tt * 16 + (l & 15);
-        if (pk >= b.rows) continue;
-        const size_t p = (size_t) b.p0 + pk;
-        const float wv = EPI == EPI_ACT ? a.wt[p] : 0.f;
+        if (pk >= rows) continue;
+        const size_t p = (size_t) p0 + pk;
+        const float wv = EPI == EPI_ACT && !SH ? a.wt[p] : 1.f;
         const int tk = EPI == EPI_FIN ? a.tok[p] : 0;
         #pragma unroll
         for (int st = 0; st < NS; ++st)
@@ -162,6 +182,61 @@ __device__ __forceinline__ void pg_store(const PgArgs& a, const Block& b, int nb
     }
 }
 
+// The input rows of a pass, staged in LDS as f16. A stage holds each tile's 16 rows x 64 k as two 1 KB blocks (row
+// halves): lane l of a block's load takes row l / 8's 16-byte chunk (l % 8) ^ (l / 8) (whole 128-byte lines from memory)
+// and lands at 16 l, so a fragment read (row l % 16, chunk 4 k + l / 16) meets distinct banks. Wave w loads half w % 2 of
+// tiles 2 j + w / 2; a pick past the block re-reads its last row (its output columns are never stored), a tile past it the
+// last tile.
+template <int NMAT, int NT, int NBUF, typename BUF>
+struct PgIn
+{
+    static constexpr int K = NMAT == 2 ? H : I, KS = K / 64, ND = (NT + 1) / 2;       // ND: stage loads per wave
+    BUF buf;
+    __amdgpu_buffer_rsrc_t xrs;
+    uint32_t src[ND];
+    int fo[2], w;
+
+    // row(p): the input row of pick p of the pass
+    template <typename ROW>
+    __device__ __forceinline__ void init(__amdgpu_buffer_rsrc_t x, int rows, ROW&& row_of)
+    {
+        const int l = threadIdx.x & 63, row = l & 15, ntt = (rows + 15) >> 4;
+        w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        xrs = x;
+        #pragma unroll
+        for (int j = 0; j < ND; ++j)
+        {
+            const int pk = min(min(2 * j + (w >> 1), ntt - 1) * 16 + 8 * (w & 1) + (l >> 3), rows - 1);
+            src[j] = (uint32_t) row_of(pk) * (K * 2) + 16 * ((l & 7) ^ (l >> 3));
+        }
+        #pragma unroll
+        for (int k = 0; k < 2; ++k) fo[k] = (row >> 3) * 64 + 8 * (l & 7) + ((4 * k + (l >> 4)) ^ (l & 7));
+    }
+    // input stage s (of a column block's KS; past the last it wraps into the next column block's) into ring buffer J: one
+    // array per buffer, or (4 buffers) two, tiles 4 .. in the second
+    template <int J> __device__ __forceinline__ void stage(int s)
+    {
+        const int so = (s >= KS ? s - KS : s) * 128;
+        #pragma unroll
+        for (int j = 0; j < ND; ++j)
+        {
+            const int tt = min(2 * j + (w >> 1), NT - 1);
+            auto put = [&](u32x4* arr, int tl) {
+                pg_load_lds(xrs, arr + (tl * 2 + (w & 1)) * 64, src[j], so);
+            };
+            if constexpr (NBUF == 8) put(buf(ic<J>{}), tt);
+            else { if (2 * j < 4) put(buf(ic<2 * J>{}), tt); else put(buf(ic<2 * J + 1>{}), tt - 4); }
+        }
+    }
+    // fragment of tile i, 32-k step k of ring buffer J
+    template <typename JC> __device__ __forceinline__ f16x8 rd(JC, int i, int k)
+    {
+        constexpr int J = JC::value;
+        if constexpr (NBUF == 8) return as_f16x8(buf(ic<J>{})[i * 128 + fo[k]]);
+        else return i < 4 ? as_f16x8(buf(ic<2 * J>{})[i * 128 + fo[k]]) : as_f16x8(buf(ic<2 * J + 1>{})[(i - 4) * 128 + fo[k]]);
+    }
+};
+
 // one pass: the picks of b (<= 16 NT) against column blocks cb0 .. cb0 + ncb of 64 NS columns, one continuous pipeline
 // (the next column block's weights and input stages load under the last groups of the one before)
 template <int EPI, int NT, int D, typename BUF>
@@ -172,30 +247,24 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
     constexpr int K = NMAT == 2 ? H : I, NOUT = NMAT == 2 ? I : H, KG = K / 128, KS = K / 64, NS = 4 / NMAT;
     constexpr int NBUF = NT <= PG_STL ? 8 : 4;              // input stages in LDS
     constexpr int WN = NT > 6 ? 2 : NT > 5 ? 3 : NT;        // input fragments held
-    constexpr int ND = (NT + 1) / 2;                        // stage loads per wave
+    constexpr int ND = (NT + 1) / 2;
     static_assert(NT % WN == 0 && KS % 8 == 0 && (D == 2 || D == 4), "the loop is unrolled over 8 stages");
     const int t = threadIdx.x, l = t & 63, row = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);   // wave index, kept in a scalar register
-    const int nb0 = (cb0 * 4 + w) * NS, ntt = (b.rows + 15) >> 4;
+    const int nb0 = (cb0 * 4 + w) * NS;
     const DqConsts dq = dq_consts();
-    // A stage holds each tile's 16 rows x 64 k as two 1 KB blocks (row halves): lane l of a block's load takes row l /
-    // 8's 16-byte chunk (l % 8) ^ (l / 8) (whole 128-byte lines from memory) and lands at 16 l, so a fragment read (row l
-    // % 16, chunk 4 k + l / 16) meets distinct banks. Wave w loads half w % 2 of tiles 2 j + w / 2; a pick past the
-    // block re-reads its last row (its output columns are never stored), a tile past it the last tile.
-    uint32_t src[ND];
-    #pragma unroll
-    for (int j = 0; j < ND; ++j)
-    {
-        const int pk = min(min(2 * j + (w >> 1), ntt - 1) * 16 + 8 * (w & 1) + (l >> 3), b.rows - 1);
+    PgIn<NMAT, NT, NBUF, BUF> in = {buf};
+    in.init(pg_rsrc((uint64_t) a.xin, (uint32_t) (NMAT == 2 ? a.T : a.np) * (K * 2)), b.rows, [&](int pk) {
         int r = b.p0 + pk;
         if (NMAT == 2)
         {
             if (a.tok) r = a.tok[r];
             r = (unsigned) r < (unsigned) a.T ? r : 0;
         }
-        src[j] = (uint32_t) r * (K * 2) + 16 * ((l & 7) ^ (l >> 3));
-    }
-    const __amdgpu_buffer_rsrc_t xrs = pg_rsrc((uint64_t) a.xin, (uint32_t) (NMAT == 2 ? a.T : a.np) * (K * 2));
+        return r;
+    });
+    auto stage = [&](int s, auto jc) { in.template stage<decltype(jc)::value>(s); };
+    auto rd = [&](auto jc, int i, int k) { return in.rd(jc, i, k); };
     __amdgpu_buffer_rsrc_t wrs[NMAT], srs[NMAT];
     #pragma unroll
     for (int m = 0; m < NMAT; ++m)
@@ -203,32 +272,6 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
         wrs[m] = pg_rsrc((uint64_t) ld_uniform((m == 0 ? a.w0 : a.w1) + b.e), NOUT * (K / 2));
         srs[m] = pg_rsrc((uint64_t) ld_uniform((m == 0 ? a.s0 : a.s1) + b.e), NOUT * KG * 2);
     }
-    int fo[2];
-    #pragma unroll
-    for (int k = 0; k < 2; ++k) fo[k] = (row >> 3) * 64 + 8 * (l & 7) + ((4 * k + (l >> 4)) ^ (l & 7));
-    // input stage s (of a column block's KS; past the last it wraps into the next column block's) into ring buffer J: one
-    // array per buffer, or (4 buffers) two, tiles 4 .. in the second
-    auto stage = [&](int s, auto jc) {
-        constexpr int J = decltype(jc)::value;
-        const int so = (s >= KS ? s - KS : s) * 128;
-        #pragma unroll
-        for (int j = 0; j < ND; ++j)
-        {
-            const int tt = min(2 * j + (w >> 1), NT - 1);
-            auto put = [&](u32x4* arr, int tl) {
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(xrs, (__attribute__((address_space(3))) void*)
-                    (arr + (tl * 2 + (w & 1)) * 64), 16, src[j], so, 0, 0);
-            };
-            if constexpr (NBUF == 8) put(buf(ic<J>{}), tt);
-            else { if (2 * j < 4) put(buf(ic<2 * J>{}), tt); else put(buf(ic<2 * J + 1>{}), tt - 4); }
-        }
-    };
-    // fragment of tile i, 32-k step k of ring buffer J
-    auto rd = [&](auto jc, int i, int k) {
-        constexpr int J = decltype(jc)::value;
-        if constexpr (NBUF == 8) return as_f16x8(buf(ic<J>{})[i * 128 + fo[k]]);
-        else return i < 4 ? as_f16x8(buf(ic<2 * J>{})[i * 128 + fo[k]]) : as_f16x8(buf(ic<2 * J + 1>{})[(i - 4) * 128 + fo[k]]);
-    };
     // the weights of group g (counted through the column blocks; past the last one its last group again) into ring slot
     // SL; when g starts a block of 4, the block's row scales too (a block's 4 bf16 of one row are 8 contiguous bytes of
     // I4G128) into sc4[SC] (SC -1: none)
@@ -277,6 +320,7 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
         {
         static_for<8>([&](auto sc8) {
             constexpr int s8 = decltype(sc8)::value, G = s8 / 2, SL = G % D;
+            constexpr int J0 = s8 % NBUF, J1 = (s8 + 1) % NBUF, JL = (s8 + NBUF - 1) % NBUF;    // ring buffers
             static_for<2>([&](auto kc) {
                 constexpr int k = decltype(kc)::value, kq = 2 * (s8 & 1) + k;       // 32-k step of the group
                 f16x8 aw[4];
@@ -307,7 +351,7 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
                     asm volatile("s_waitcnt vmcnt(%0)" :: "n"(after) : "memory");
                     __builtin_amdgcn_s_barrier();
                     __builtin_amdgcn_sched_barrier(0);
-                    stage(s0 + s8 + NBUF - 1, ic<(s8 + NBUF - 1) % NBUF>{});
+                    stage(s0 + s8 + NBUF - 1, ic<JL>{});
                     // on odd stages the group's ring slot is consumed: refill it D groups ahead
                     if constexpr (s8 & 1) fetch(c * KG + s0 / 2 + G + D, ic<SL>{}, ic<(G + D) % 4 == 0 ? 1 : -1>{});
                     __builtin_amdgcn_sched_barrier(0);
@@ -318,8 +362,8 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
                     #pragma unroll
                     for (int f = 0; f < 4; ++f) acc[f][i] = mfma16(aw[f], bq[i % WN], acc[f][i]);
                     // the fragment WN tiles on: of this step, or of the next one
-                    if (i + WN < NT) bq[i % WN] = rd(ic<s8 % NBUF>{}, i + WN, k);
-                    else bq[i % WN] = k == 0 ? rd(ic<s8 % NBUF>{}, i + WN - NT, 1) : rd(ic<(s8 + 1) % NBUF>{}, i + WN - NT, 0);
+                    if (i + WN < NT) bq[i % WN] = rd(ic<J0>{}, i + WN, k);
+                    else bq[i % WN] = k == 0 ? rd(ic<J0>{}, i + WN - NT, 1) : rd(ic<J1>{}, i + WN - NT, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             });
@@ -330,9 +374,102 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
             }
         });
         }
-        pg_store<EPI, NT>(a, b, nb0 + c * (4 * NS), l, acc);
+        pg_store<EPI, NT, false>(a, b.p0, b.rows, nb0 + c * (4 * NS), l, acc);
     }
     // (no stage load may land in LDS after the workgroup has given it up)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// A pass of the shared expert, merged into the routed launches: by itself it was two dense launches whose few workgroups
+// were a chain of 96 and 32 serial stages (83 + 25 us from 17 to ~500 tokens, 104 + 64 at 2048); here that chain runs beside
+// the routed blocks (33 tokens: 706 -> 639 us per layer; 150: 993 -> 935; 1000: 1311 -> 1263; 2048: 1815 -> 1796).
+// tokens t0 .. t0 + rows (<= 16 NT) against column blocks cb0 .. cb0 + ncb. As pg_pass with the
+// f16 weights loaded as fragments (16 rows x 64 bytes) into a ring of DS 64-k stages, each refilled one step after its
+// last use; the k order of every sum is that of a 32-k chain, as everywhere.
+template <int EPI, int NT, int DS, typename BUF>
+__device__ __forceinline__ void pg_dense(BUF buf, const PgArgs& a, int t0, int rows, int cb0, int ncb_)
+{
+    constexpr int NMAT = EPI == EPI_ACT ? 2 : 1;
+    const int ncb = NMAT == 2 ? 1 : ncb_;
+    constexpr int K = NMAT == 2 ? H : I, NOUT = NMAT == 2 ? I : H, KS = K / 64, NS = 4 / NMAT;
+    constexpr int NBUF = NT <= PG_STL ? 8 : 4, WN = NT > 6 ? 2 : NT > 5 ? 3 : NT, ND = (NT + 1) / 2;
+    static_assert(NT % WN == 0 && KS % 8 == 0 && 8 % DS == 0, "the loop is unrolled over 8 stages");
+    const int l = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nb0 = (cb0 * 4 + w) * NS, r0 = NMAT == 2 ? t0 : a.ps + t0;                // first input row
+    PgIn<NMAT, NT, NBUF, BUF> in = {buf};
+    in.init(pg_rsrc((uint64_t) a.xin, (uint32_t) (NMAT == 2 ? a.T : a.ps + a.T) * (K * 2)), rows,
+            [&](int pk) { return r0 + pk; });
+    auto stage = [&](int s, auto jc) { in.template stage<decltype(jc)::value>(s); };
+    auto rd = [&](auto jc, int i, int k) { return in.rd(jc, i, k); };
+    __amdgpu_buffer_rsrc_t wrs[NMAT];
+    #pragma unroll
+    for (int m = 0; m < NMAT; ++m) wrs[m] = pg_rsrc((uint64_t) (m == 0 ? a.sh0 : a.sh1), NOUT * K * 2);
+    const int wo = (l & 15) * (K * 2) + 16 * (l >> 4);
+    // the weights of stage s (counted through the column blocks; past the last one its last stage again) into slot SL
+    u32x4 ring[DS][2][4];
+    auto fetch = [&](int s, auto sl) {
+        constexpr int SL = decltype(sl)::value;
+        const int sc = min(s, ncb * KS - 1), c = sc / KS, sk = sc - c * KS;
+        #pragma unroll
+        for (int k = 0; k < 2; ++k)
+            #pragma unroll
+            for (int f = 0; f < 4; ++f)
+                ring[SL][k][f] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wrs[f % NMAT], wo,
+                    (nb0 + c * (4 * NS) + f / NMAT) * (16 * K * 2) + (2 * sk + k) * 64, 0));
+    };
+    f32x4 acc[4][NT];
+    static_for<DS - 1>([&](auto g) {
+        fetch(decltype(g)::value, g);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    static_for<NBUF - 1>([&](auto j) {
+        stage(decltype(j)::value, j);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    f16x8 bq[WN];
+    #pragma unroll
+    for (int i = 0; i < WN; ++i) bq[i] = rd(ic<0>{}, i, 0);
+    for (int c = 0; c < ncb; ++c)
+    {
+        #pragma unroll
+        for (int f = 0; f < 4; ++f)
+            #pragma unroll
+            for (int i = 0; i < NT; ++i) acc[f][i] = (f32x4) {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = 0; s0 < KS; s0 += 8)
+            static_for<8>([&](auto sc8) {
+                constexpr int s8 = decltype(sc8)::value, SL = s8 % DS;
+                constexpr int J0 = s8 % NBUF, J1 = (s8 + 1) % NBUF, JL = (s8 + NBUF - 1) % NBUF;
+                static_for<2>([&](auto kc) {
+                    constexpr int k = decltype(kc)::value;
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (k == 0) fetch(c * KS + s0 + s8 + DS - 1, ic<(s8 + DS - 1) % DS>{});
+                    else
+                    {
+                        // the next stage, as in pg_pass: older than the stage loads of the last NBUF - 3 bundles and the 8
+                        // weight loads of each of the last NBUF - 2 stages
+                        asm volatile("s_waitcnt vmcnt(%0)" :: "n"((NBUF - 3) * ND + (NBUF - 2) * 8) : "memory");
+                        __builtin_amdgcn_s_barrier();
+                        __builtin_amdgcn_sched_barrier(0);
+                        stage(s0 + s8 + NBUF - 1, ic<JL>{});
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    #pragma unroll
+                    for (int i = 0; i < NT; ++i)
+                    {
+                        #pragma unroll
+                        for (int f = 0; f < 4; ++f) acc[f][i] = mfma16(as_f16x8(ring[SL][k][f]), bq[i % WN], acc[f][i]);
+                        if (i + WN < NT) bq[i % WN] = rd(ic<J0>{}, i + WN, k);
+                        else bq[i % WN] = k == 0 ? rd(ic<J0>{}, i + WN - NT, 1) : rd(ic<J1>{}, i + WN - NT, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                });
+            });
+        pg_store<EPI, NT, true>(a, a.ps + t0, rows, nb0 + c * (4 * NS), l, acc);
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
@@ -354,8 +491,32 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     };
     constexpr int NMAT = EPI == EPI_ACT || EPI == EPI_RAW ? 2 : 1;
     constexpr int NCB = (NMAT == 2 ? I : H) / (256 / NMAT);
+    const int ny = NCB / a.ncb;
+    int i = blockIdx.x;
+    if constexpr (EPI == EPI_ACT || EPI == EPI_D16)
+    {
+        // the shared expert's blocks come first: they are the longest, and the rest fills in around them. The token blocks of
+        // one column block go to consecutive workgroups of one XCD, which then reads its weights once.
+        const int ns = a.nsh * ny;
+        if (i < ns)
+        {
+            const int j = i >> 3;
+            const int cb = (ny & 7) == 0 ? (j / a.nsh) * 8 + (i & 7) : i / a.nsh;
+            const int t0 = ((ny & 7) == 0 ? j : i) % a.nsh * a.sh_rows, rows = min(a.sh_rows, a.T - t0);
+            if (rows <= 0) return;
+            switch ((rows + 31) >> 5)
+            {
+                case 1: pg_dense<EPI, 2, 4>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
+                case 2: pg_dense<EPI, 4, 4>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
+                case 3: pg_dense<EPI, 6, 2>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
+                default: pg_dense<EPI, 8, 2>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
+            }
+            return;
+        }
+        i -= ns;
+    }
     int rbi, cbi;
-    xcd_tile(rbi, cbi, (a.nrb + 7) & ~7, NCB / a.ncb);
+    xcd_tile(i, rbi, cbi, ny);
     Block rb;
     if (!get_block(a.rbt, a.nrb, a.meta, a.n_tab, a.np, rbi, rb)) return;
     // a block of more than PG_PB picks runs as passes, one after the other (a later pass reads the weights again,

@@ -11,7 +11,9 @@ int hmoe::grouped_down(const PgArgs& a, int epi, hipStream_t st)
     // 133 us; equal at about 25 tokens).
     PgArgs g = a;
     g.ncb = a.np < 200 ? 2 : 3;
-    const dim3 grid = pgemm_grid(a.nrb, H / 256 / g.ncb);
+    pg_shared_blocks(g);
+    const dim3 grid(pgemm_grid(a.nrb, H / 256 / g.ncb).x + g.nsh * (H / 256 / g.ncb));
+    if (grid.x == 0) return HMOE_OK;
     if (epi == EPI_D16) pgemm_kernel<EPI_D16><<<grid, 256, 0, st>>>(g);
     else if (epi == EPI_FIN) pgemm_kernel<EPI_FIN><<<grid, 256, 0, st>>>(g);
     else pgemm_kernel<EPI_D><<<grid, 256, 0, st>>>(g);

@@ -7,7 +7,9 @@ int hmoe::grouped_gate_up(const PgArgs& a, int epi, hipStream_t st)
 {
     PgArgs g = a;
     g.ncb = 1;
-    const dim3 grid = pgemm_grid(a.nrb, I / 128);
+    pg_shared_blocks(g);
+    const dim3 grid(pgemm_grid(a.nrb, I / 128).x + g.nsh * (I / 128));
+    if (grid.x == 0) return HMOE_OK;
     if (epi == EPI_ACT) pgemm_kernel<EPI_ACT><<<grid, 256, 0, st>>>(g);
     else pgemm_kernel<EPI_RAW><<<grid, 256, 0, st>>>(g);
     return HMOE_LAUNCHED("grouped gate/up");

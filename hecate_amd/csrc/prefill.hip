@@ -6,7 +6,7 @@
 // GEMMs: workgroup = (row block of picks of one expert, 128 gate/up or 256 down output columns); see pgemm.h, and
 // pgemm16_kernel for the long prefill. gu fuses act = silu(g) * u * w (f16), down writes d = W_d act (fp32), fin adds each
 // token's picks into out in top-k order (or with atomics, as p4_fin_kernel, when no inverse map is given). The shared
-// expert's projections run on the dense MFMA GEMMs of shared_gemm.hip.
+// expert's projections ride in the same launches (moe4p) or run on the dense MFMA GEMMs of shared_gemm.hip.
 #include "pgemm.h"
 
 namespace hmoe {
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2
     __shared__ __attribute__((aligned(16))) u32x4 xs0[NTT * 4 * 64];
     __shared__ __attribute__((aligned(16))) u32x4 xs1[NTT * 4 * 64];
     int rbi, cbi;
-    xcd_tile(rbi, cbi, (nrb + 7) & ~7, NOUT / (16 * NS * NWV));
+    xcd_tile(blockIdx.x, rbi, cbi, NOUT / (16 * NS * NWV));
     Block rb;
     if (!get_block(rbt, nrb, meta, n_tab, np, rbi, rb)) return;
     // a block of more than PBX picks runs as passes of PBX, one after the other (a later pass reads the weights
@@ -561,6 +561,8 @@ static int moe4p_run(const void* x, const int* tok, const float* wt, const int* 
                  "moe4p_forward: tables");
     HMOE_REQUIRE((!sh_gw && !sh_uw && !sh_dw) || (sh_gw && sh_uw && sh_dw && inv),
                  "moe4p_forward: the shared expert needs all three matrices and the inverse map");
+    HMOE_REQUIRE((((uintptr_t) sh_gw | (uintptr_t) sh_uw | (uintptr_t) sh_dw) & 15) == 0,
+                 "moe4p_forward: the shared expert's matrices are 16-byte aligned");
     HMOE_REQUIRE(((uintptr_t) x & 15) == 0 && ((uintptr_t) ar & 15) == 0 && ((uintptr_t) d & 15) == 0 &&
                  ((uintptr_t) out & 15) == 0, "moe4p_forward: alignment");
     HMOE_REQUIRE(xf == HMOE_XF_BF16 || xf == HMOE_XF_F16, "moe4p_forward: xf must be HMOE_XF_BF16 (0) or HMOE_XF_F16 "
@@ -576,29 +578,19 @@ static int moe4p_run(const void* x, const int* tok, const float* wt, const int* 
     _Float16* a = (_Float16*) ar;
     // gate/up, then down into d rows for the ordered combine (inv given) or added into out[tok] by its epilogue (no
     // inverse map: the atomic combine of p4_fin_kernel)
-    if (nrb > 0)
-    {
-        PgArgs g{};
-        g.xin = (const _Float16*) xb; g.tok = tok; g.wt = wt; g.rbt = rbt; g.meta = meta;
-        g.w0 = gw; g.w1 = uw; g.s0 = gs; g.s1 = us; g.out = a;
-        g.nrb = nrb; g.n_tab = n_tab; g.T = T; g.np = npos; g.ps = ps;
-        if (int rc = grouped_gate_up(g, EPI_ACT, st)) return rc;
-        g.xin = a; g.w0 = dw; g.s0 = ds; g.w1 = g.s1 = nullptr;
-        g.out = inv ? d : out;
-        if (int rc = grouped_down(g, inv ? EPI_D16 : EPI_FIN, st)) return rc;
-    }
+    // The shared expert (every token) rides in the same two launches: act rows ps.. = f16(silu(gate x) up x), then down
+    // into d rows ps.. (f16), which the ordered combine adds after each token's picks
     const bool sh = sh_gw != nullptr;
-    if (sh)
-    {
-        // the shared expert on every token: act rows ps.. = f16(silu(gate x) up x), then down into d rows ps.. (f16),
-        // which the ordered combine adds after each token's picks
-        if (int rc = dense_gate_up((const _Float16*) sh_gw, (const _Float16*) sh_uw, (const _Float16*) xb, T,
-                                   a + (size_t) ps * I, st))
-            return rc;
-        if (int rc = dense_down((const _Float16*) sh_dw, a + (size_t) ps * I, T, (_Float16*) d + (size_t) ps * H,
-                                DG_MODE_F16, st))
-            return rc;
-    }
+    PgArgs g{};
+    g.xin = (const _Float16*) xb; g.tok = tok; g.wt = wt; g.rbt = rbt; g.meta = meta;
+    g.w0 = gw; g.w1 = uw; g.s0 = gs; g.s1 = us; g.out = a;
+    g.nrb = nrb; g.n_tab = n_tab; g.T = T; g.np = npos; g.ps = ps;
+    g.sh0 = (const _Float16*) sh_gw; g.sh1 = (const _Float16*) sh_uw;
+    if (int rc = grouped_gate_up(g, EPI_ACT, st)) return rc;
+    g.xin = a; g.w0 = dw; g.s0 = ds; g.w1 = g.s1 = nullptr;
+    g.sh0 = (const _Float16*) sh_dw; g.sh1 = nullptr;
+    g.out = inv ? d : out;
+    if (int rc = grouped_down(g, inv ? EPI_D16 : EPI_FIN, st)) return rc;
     if (inv && ob) pfin_kernel<PF_BF16><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, sh ? ps : -1, nullptr, ob);
     else if (inv) pfin_kernel<PF_ADD><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, sh ? ps : -1, out, nullptr);
     return HMOE_LAUNCHED("moe4p_forward");
@@ -664,7 +656,7 @@ extern "C" int hmoe_shared_forward(const void* x, int T, const void* sh_gw, cons
     _Float16* a = (_Float16*) (wk + shw_act(T));
     if (int rc = dense_gate_up((const _Float16*) sh_gw, (const _Float16*) sh_uw, xs, T, a, st)) return rc;
     // (out += each product element once, in the GEMM's epilogue)
-    if (int rc = dense_down((const _Float16*) sh_dw, a, T, out, DG_MODE_ADD, st)) return rc;
+    if (int rc = dense_down((const _Float16*) sh_dw, a, T, out, st)) return rc;
     return HMOE_LAUNCHED("shared_forward");
 }
 

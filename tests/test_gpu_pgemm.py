@@ -1,5 +1,6 @@
 """The grouped expert GEMM at every pick-tile count and its edges: one expert with n picks (and a neighbour with 3), through
-the device dispatch and moe4p.forward, against a torch fp32 reference on the same dequantised weights."""
+the device dispatch and moe4p.forward, against a torch fp32 reference on the same dequantised weights; and the shared
+expert in the same launches at the edges of its token blocks."""
 import pytest
 import torch
 
@@ -11,7 +12,15 @@ NS = (1, 15, 16, 17, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 112, 113, 128, 129,
 @pytest.fixture(scope="module")
 def lay():
     from hecate_amd import synth
-    return synth.make_layer(0, torch.device("cuda:0"), resident=[3, 7], shared=False)
+    return synth.make_layer(0, torch.device("cuda:0"), resident=[3, 7])
+
+
+def bound(ref):
+    # the act rows are rounded to f16: each of the 2048 terms of an output carries an independent error of at most 2^-11 of
+    # it, so the output's error has a standard deviation of at most 2^-11 of the row's rms (the act row is heavy-tailed: a
+    # few terms make most of it, so the bound of one rounding is taken, not its average); five of those for the largest of
+    # ~10^6 outputs, and, ordered, the down row is rounded once more
+    return 5 * 2.0 ** -11 * ref.square().mean(1, keepdim=True).sqrt() + (2.0 ** -11) * ref.abs()
 
 
 @pytest.mark.parametrize("ordered", (True, False))
@@ -32,10 +41,29 @@ def test_pick_counts(lay, n, bm, ordered):
     moe4p.forward(x, pf.tok, pf.eid, pf.wt, pf.rbt, gq, uq, dq, gs, us, ds, *pf.scr, y,
                   inv=pf.inv if ordered else None, meta=pf.meta, topk=1, npos=T, nrb=pf.nrb_max)
     ref = moe_rows(lay, x, sel, rw, with_shared=False)
-    # the act rows are rounded to f16: each of the 2048 terms of an output carries an independent error of at most 2^-11 of
-    # it, so the output's error has a standard deviation of at most 2^-11 of the row's rms (the act row is heavy-tailed: a
-    # few terms make most of it, so the bound of one rounding is taken, not its average); five of those for the largest of
-    # ~10^6 outputs, and, ordered, the down row is rounded once more
-    bound = 5 * 2.0 ** -11 * ref.square().mean(1, keepdim=True).sqrt() + (2.0 ** -11) * ref.abs()
-    worst = ((y - ref).abs() / bound).max().item()
+    worst = ((y - ref).abs() / bound(ref)).max().item()
     assert worst <= 1.0, (n, bm, ordered, worst)
+
+
+@pytest.mark.parametrize("T", (1, 16, 17, 32, 33, 64, 65, 96, 97, 128, 129, 130, 256, 257, 300))
+def test_shared_blocks(lay, T):
+    from hecate_amd import moe4p, synth, tier
+    from torchref import moe_rows
+    dev = lay.device
+    x = synth.gen_x(400 + T, T, dev)
+    sel = torch.full((T, 1), 2, dtype=torch.int64, device=dev)            # outside the window, but for a few tokens
+    sel[::5] = 0
+    rw = torch.full((T, 1), 0.5, dtype=torch.float16, device=dev)
+    pf = tier.PrefillBuffers(T, 1, 0, 2, 256, dev).run(sel, rw)
+    out = torch.empty((T, 6144), dtype=torch.bfloat16, device=dev)
+    y = torch.zeros((T, 6144), dtype=torch.float32, device=dev)
+    gq, uq, dq, gs, us, ds = lay.bank.tables()
+    a = (x, pf.tok, pf.eid, pf.wt, pf.rbt, gq, uq, dq, gs, us, ds, *pf.scr)
+    kw = dict(inv=pf.inv, meta=pf.meta, topk=1, npos=T, nrb=pf.nrb_max, shared=lay.shared_rows())
+    moe4p.forward(*a, y, **kw)
+    moe4p.forward(*a, None, out_bf16=out, **kw)
+    routed = moe_rows(lay, x, sel, rw, with_shared=False)
+    ref = moe_rows(lay, x, sel, rw)
+    worst = ((y - ref).abs() / (bound(ref - routed) + bound(routed).clamp_min(1e-30))).max().item()
+    assert worst <= 1.0, (T, worst)
+    assert torch.equal(out.view(torch.int16), y.bfloat16().view(torch.int16))
