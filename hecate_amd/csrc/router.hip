@@ -5,8 +5,9 @@
 //   small (R <= 16): a logits kernel (two experts per workgroup, one 32-element chunk per thread, chunk sums folded
 //                    through LDS) and a select kernel (one wave per row); the kernel boundary replaces the reference's
 //                    last-block counter (exl3_router.py:74-83,130), whose cross-workgroup fences are costly on gfx950.
-//   large (R > 16) : an fp32 MFMA GEMM per (128 rows, 64 experts, segment) with the same chain order, then a select
-//                    kernel that folds the 8 segment sums and picks each row's top-k (one wave per row).
+//   large (R > 16) : an fp32 MFMA GEMM per (row tile, expert tile, segment) with the same chain order (one wave per tile up
+//                    to SR_ROWS rows, 128 rows x 64 experts per workgroup above), then a select kernel that folds the 8
+//                    segment sums and picks each row's top-k (one wave per row).
 #include "hmoe_dev.h"
 
 namespace hmoe {
@@ -149,22 +150,161 @@ __global__ void __launch_bounds__(256) router_seg_mfma_kernel(
         }
 }
 
+// The same up to SR_ROWS rows, where the kernel above is a few workgroups of 24 serial chunks, a barrier each. One wave owns 16 NR rows x 16 NE experts of one segment and needs no LDS and no
+// barrier: lane l loads k 8(l/16) .. + 8 of row (expert) l % 16 of a chunk - 16 bytes of x, 32 of w - and a 4 x 4 transpose
+// between the four 16-lane groups (two permlane16 and two permlane32 swaps per four registers) gives each MFMA step its
+// operand, k 4 kk + l/16. The loads run D - 1 chunks ahead of their use.
+// What bounds it: the load latency of the 24 serial chunks. Router with its select, 256 experts, same bits: 33 rows 49.6 ->
+// 18.0 us, 150 rows 50.2 -> 26.1, 450 rows 53.8 -> 32.5.
+constexpr int SR_ROWS = 768;
+template <int NR, int NE>
+struct SegChunk { u32x4 x[NR]; f32x4 w[NE][2]; };
+
+// registers v[0..3] of lane group g holding elements 0..3 of quad g -> v[i] of lane group g = element g of quad i
+__device__ __forceinline__ void transpose4(float (&v)[4])
+{
+    auto swap16 = [](float& a, float& b) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+    };
+    auto swap32 = [](float& a, float& b) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        a = __uint_as_float(r[0]); b = __uint_as_float(r[1]);
+    };
+    swap16(v[0], v[1]); swap16(v[2], v[3]);
+    swap32(v[0], v[2]); swap32(v[1], v[3]);
+}
+
+// workgroup: 4 waves = 4 expert groups of one row tile; blockIdx.x: row tile x (experts / (64 NE) rounded up), y: segment
+template <int NR, int NE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) router_seg_wave_kernel(
+    const uint16_t* __restrict__ x, const float* __restrict__ wt, float* __restrict__ seg, int R, int K, int E, int ney)
+{
+    constexpr int D = 4;
+    const int l = threadIdx.x & 63, g = l >> 4, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r0 = (blockIdx.x / ney) * 16 * NR, e0 = ((blockIdx.x % ney) * 4 + w) * 16 * NE, s = blockIdx.y;
+    if (e0 >= E) return;                                        // (no barrier in this kernel)
+    const int segk = K / RSEG, k0 = s * segk, nch = segk / RCHUNK;
+    const uint16_t* xp[NR];
+    const float* wp[NE];
+    #pragma unroll
+    for (int i = 0; i < NR; ++i) xp[i] = x + (size_t) min(r0 + 16 * i + (l & 15), R - 1) * K + k0 + 8 * g;
+    #pragma unroll
+    for (int j = 0; j < NE; ++j) wp[j] = wt + (size_t) min(e0 + 16 * j + (l & 15), E - 1) * K + k0 + 8 * g;
+    SegChunk<NR, NE> ring[D];
+    auto load = [&](SegChunk<NR, NE>& q, int c) {
+        const int o = min(c, nch - 1) * RCHUNK;
+        #pragma unroll
+        for (int i = 0; i < NR; ++i) q.x[i] = *(const u32x4*) (xp[i] + o);
+        #pragma unroll
+        for (int j = 0; j < NE; ++j)
+        {
+            q.w[j][0] = *(const f32x4*) (wp[j] + o);
+            q.w[j][1] = *(const f32x4*) (wp[j] + o + 4);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    f32x4 tot[NR][NE];
+    #pragma unroll
+    for (int i = 0; i < NR; ++i)
+        #pragma unroll
+        for (int j = 0; j < NE; ++j) tot[i][j] = (f32x4) {0.f, 0.f, 0.f, 0.f};
+    auto chunk = [&](const SegChunk<NR, NE>& q) {
+        f32x4 d[NR][NE];
+        // operands of MFMA step kk: quad kk = 2 i + h is register i of set h (quads 2 g + h of the four lane groups)
+        float a[NR][2][4], b[NE][2][4];
+        #pragma unroll
+        for (int i = 0; i < NR; ++i)
+            #pragma unroll
+            for (int h = 0; h < 2; ++h)
+            {
+                #pragma unroll
+                for (int p = 0; p < 2; ++p)
+                {
+                    a[i][h][2 * p] = __uint_as_float(q.x[i][2 * h + p] << 16);
+                    a[i][h][2 * p + 1] = __uint_as_float(q.x[i][2 * h + p] & 0xffff0000u);
+                }
+                transpose4(a[i][h]);
+            }
+        #pragma unroll
+        for (int j = 0; j < NE; ++j)
+            #pragma unroll
+            for (int h = 0; h < 2; ++h)
+            {
+                #pragma unroll
+                for (int p = 0; p < 4; ++p) b[j][h][p] = q.w[j][h][p];
+                transpose4(b[j][h]);
+            }
+        #pragma unroll
+        for (int kk = 0; kk < RCHUNK / 4; ++kk)
+            #pragma unroll
+            for (int i = 0; i < NR; ++i)
+                #pragma unroll
+                for (int j = 0; j < NE; ++j)
+                    d[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][kk & 1][kk >> 1], b[j][kk & 1][kk >> 1],
+                                                                   kk == 0 ? (f32x4) {0.f, 0.f, 0.f, 0.f} : d[i][j],
+                                                                   0, 0, 0);
+        #pragma unroll
+        for (int i = 0; i < NR; ++i)
+            #pragma unroll
+            for (int j = 0; j < NE; ++j) tot[i][j] = tot[i][j] + d[i][j];
+    };
+    static_for<D - 1>([&](auto c) { load(ring[decltype(c)::value], decltype(c)::value); });
+    for (int c0 = 0; c0 < nch; c0 += D)
+        static_for<D>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            load(ring[(c + D - 1) % D], c0 + c + D - 1);
+            if (c0 + c < nch) chunk(ring[c]);
+        });
+    #pragma unroll
+    for (int i = 0; i < NR; ++i)
+        #pragma unroll
+        for (int q = 0; q < 4; ++q)
+        {
+            const int r = r0 + 16 * i + 4 * g + q;
+            if (r >= R) continue;
+            #pragma unroll
+            for (int j = 0; j < NE; ++j)
+            {
+                const int e = e0 + 16 * j + (l & 15);
+                if (e < E) seg[((size_t) s * R + r) * RMAXE + e] = tot[i][j][q];
+            }
+        }
+}
+
+template <int NR, int NE>
+static void router_seg(const uint16_t* x, const float* wt, float* seg, int R, int K, int E, hipStream_t st)
+{
+    const int ney = (E + 64 * NE - 1) / (64 * NE);
+    router_seg_wave_kernel<NR, NE><<<dim3((R + 16 * NR - 1) / (16 * NR) * ney, RSEG), 256, 0, st>>>(x, wt, seg, R, K, E, ney);
+}
+
 // large path, 2: fold the segments in order, select; one wave per row; optional f16 copy of x
 __global__ void __launch_bounds__(256) router_select_kernel(const float* __restrict__ seg, const float* __restrict__ bias,
     int R, int E, int topk, float scale, int64_t* __restrict__ sel, uint16_t* __restrict__ rw,
     const uint16_t* __restrict__ x, _Float16* __restrict__ xh, int K)
 {
-    __shared__ float lrow[4][RMAXE];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + wave;
     if (r >= R) return;
-    for (int e = lane; e < E; e += 64)
+    // (every plane's loads and the bias in flight together, then the sums in segment order)
+    RowIn in;
+    float v[4][RSEG];
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
+        #pragma unroll
+        for (int s = 0; s < RSEG; ++s)
+            v[i][s] = ldg<float>(seg + ((size_t) s * R + r) * RMAXE + min(lane + 64 * i, E - 1));
+    load_bias_global(bias, seg, E, in.b);
+    #pragma unroll
+    for (int i = 0; i < 4; ++i)
     {
-        float t = 0.f;
-        for (int s = 0; s < RSEG; ++s) t = t + seg[((size_t) s * R + r) * RMAXE + e];
-        lrow[wave][e] = t;
+        in.lg[i] = 0.f;
+        #pragma unroll
+        for (int s = 0; s < RSEG; ++s) in.lg[i] = in.lg[i] + v[i][s];
     }
-    select_row(lrow[wave], bias, E, topk, scale, sel + (size_t) r * topk, rw + (size_t) r * topk);
+    bias_or_zero(in.b, bias != nullptr);
+    select_from(in, E, topk, scale, sel + (size_t) r * topk, rw + (size_t) r * topk);
     if (xh)
         for (int k = lane * 8; k < K; k += 64 * 8)
         {
@@ -215,10 +355,17 @@ extern "C" int hmoe_router_fused(const void* x, const float* wt, const float* bi
         if (int rc = HMOE_LAUNCHED("router_fused")) return rc;
         return router_select_small(logits, bias, R, E, topk, scale, sel, rw, st);
     }
-    // 128 experts per workgroup from 4096 rows (the 8 x 8 tiles are faster at 8192 rows, -115 us); fewer rows take 64
-    // experts per workgroup, so that the grid still fills the CUs twice over
-    router_seg_mfma_kernel<<<dim3((R + SM_R - 1) / SM_R, (E + SM_E - 1) / SM_E, RSEG), 256, 0, st>>>(
-            (const uint16_t*) x, wt, logits, R, K, E);
+    // Small tiles while the launch would not fill the chip otherwise (measured with the select, us: 64 rows 18.1 with 16 x 16
+    // per wave, 24.3 with 16 x 32; 150 rows 27.5, 26.1 and 30.5 with 32 x 32; 450 rows 47.7, 41.7, 32.5). From ~700 rows the
+    // LDS-staged tiles reuse their operands more (700 rows 54.5 against 52.1, 1000 rows 54.7 against 53.5, 2048 rows 83
+    // against 95).
+    const uint16_t* xb = (const uint16_t*) x;
+    if (R <= 96) router_seg<1, 1>(xb, wt, logits, R, K, E, st);
+    else if (R <= 320) router_seg<1, 2>(xb, wt, logits, R, K, E, st);
+    else if (R <= SR_ROWS) router_seg<2, 2>(xb, wt, logits, R, K, E, st);
+    else
+        router_seg_mfma_kernel<<<dim3((R + SM_R - 1) / SM_R, (E + SM_E - 1) / SM_E, RSEG), 256, 0, st>>>(xb, wt, logits, R, K,
+                                                                                                       E);
     router_select_kernel<<<(R + 3) / 4, 256, 0, st>>>(logits, bias, R, E, topk, scale, sel, rw, (const uint16_t*) x,
                                                       (_Float16*) xh, K);
     return HMOE_LAUNCHED("router_fused");
