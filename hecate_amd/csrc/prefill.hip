@@ -39,6 +39,20 @@ __global__ void __launch_bounds__(DBLK) disp_count_kernel(const int64_t* __restr
     if (t < n) hist[(size_t) blockIdx.x * n + t] = h[t];
 }
 
+// the row blocks of expert e: its c picks from position first as nb blocks of at most bm, rows rb0 .. of the table
+__device__ __forceinline__ void disp_blocks(int e, int c, int nb, int bm, int balance, int first, int rb0,
+                                            int* __restrict__ rbt, int nrb_max)
+{
+    for (int k = 0; k < nb; ++k)
+    {
+        int rows, start;
+        if (balance) { const int bs = c / nb, ex = c % nb; rows = bs + (k < ex ? 1 : 0); start = k * bs + (k < ex ? k : ex); }
+        else { rows = min(bm, c - bm * k); start = bm * k; }
+        const int r = rb0 + k;
+        if (r < nrb_max) { rbt[4 * r + 0] = e; rbt[4 * r + 1] = first + start; rbt[4 * r + 2] = rows; rbt[4 * r + 3] = 0; }
+    }
+}
+
 // the per-block histograms -> each block's first position per expert (hist rewritten in place), the expert counts,
 // the row-block table and meta. Thread (q, e) of 4 x 256 covers a quarter of the blocks for expert e, its loads
 // issued 8 at a time so that they are in flight together (a load-add-store chain over the blocks waits out one load
@@ -102,14 +116,7 @@ __global__ void __launch_bounds__(1024) disp_scan_kernel(int* __restrict__ hist,
     if (q == 0 && live)
     {
         counts[e] = c;
-        for (int k = 0; k < nb; ++k)
-        {
-            int rows, start;
-            if (balance) { const int bs = c / nb, ex = c % nb; rows = bs + (k < ex ? 1 : 0); start = k * bs + (k < ex ? k : ex); }
-            else { rows = min(bm, c - bm * k); start = bm * k; }
-            const int r = rb0 + k;
-            if (r < nrb_max) { rbt[4 * r + 0] = e; rbt[4 * r + 1] = off_e + start; rbt[4 * r + 2] = rows; rbt[4 * r + 3] = 0; }
-        }
+        disp_blocks(e, c, nb, bm, balance, off_e, rb0, rbt, nrb_max);
     }
     if (threadIdx.x == 255) { meta[0] = sc[255]; meta[1] = min(sr[255], nrb_max); meta[2] = sr[255]; meta[3] = 0; }
 }
@@ -125,6 +132,99 @@ __global__ void __launch_bounds__(DBLK) disp_place_kernel(const int64_t* __restr
     const int e = (int) v;
     const int p = hist[(size_t) blockIdx.x * n + e] + rank[i];
     tok[p] = i / topk; eid[p] = e; wt[p] = (float) __builtin_bit_cast(_Float16, rw[i]); inv[i] = p;
+}
+
+// The whole plan of up to DS_PICKS picks in one launch of one workgroup: the three launches above are launch boundaries and
+// latency for a few thousand picks (8 picks a token, 256 experts: 33 tokens 12.8 -> 7.8 us, 300 tokens 13.5 -> 8.6, 512
+// tokens 13.1 -> 10.7). Past DS_PICKS one CU is slower (1000 tokens 13.7 us in three launches, 20.8 in one). Wave w owns a
+// contiguous 16th of the picks in rounds of 64 in order; in a round a lane's rank among the picks of its expert is the
+// number of lower lanes with the same expert (8 ballots over the id's bits) plus the wave's count so far, so the order is
+// that of the three launches: stable by flat index.
+constexpr int DS_W = 16, DS_RND = 4, DS_PICKS = DS_W * DS_RND * 64;
+__global__ void __launch_bounds__(DS_W * 64) disp_one_kernel(
+    const int64_t* __restrict__ sel, const uint16_t* __restrict__ rw, int F, int topk, int lo, int n, int bm, int balance,
+    int* __restrict__ counts, int* __restrict__ tok, int* __restrict__ eid, float* __restrict__ wt, int* __restrict__ inv,
+    int* __restrict__ rbt, int nrb_max, int* __restrict__ meta)
+{
+    __shared__ int hist[DS_W][256];                             // the wave's picks of each expert; then their first positions
+    __shared__ int wc[4], wb[4];
+    const int t = threadIdx.x, l = t & 63, w = t >> 6;
+    for (int i = t; i < DS_W * 256; i += DS_W * 64) (&hist[0][0])[i] = 0;
+    const int rounds = (F + DS_W * 64 - 1) / (DS_W * 64), p0 = w * rounds * 64;     // (rounds <= DS_RND)
+    int e[DS_RND], rk[DS_RND];
+    uint16_t wv[DS_RND];
+    #pragma unroll
+    for (int r = 0; r < DS_RND; ++r)
+    {
+        const int p = min(p0 + 64 * r + l, F - 1);
+        e[r] = -1; wv[r] = 0;
+        if (r < rounds)
+        {
+            const int64_t v = sel[p] - lo;
+            wv[r] = rw[p];
+            e[r] = p0 + 64 * r + l < F && v >= 0 && v < n ? (int) v : -1;
+        }
+    }
+    __syncthreads();
+    const uint64_t below = (1ull << l) - 1;
+    #pragma unroll
+    for (int r = 0; r < DS_RND; ++r)
+        if (r < rounds)
+        {
+            const bool live = e[r] >= 0;
+            uint64_t m = __ballot(live);
+            #pragma unroll
+            for (int b = 0; b < 8; ++b)
+            {
+                const uint64_t s = __ballot((e[r] >> b) & 1);
+                m &= (e[r] >> b) & 1 ? s : ~s;
+            }
+            // (the wave's own LDS reads and writes take effect in issue order; the fence keeps the compiler's)
+            const int base = live ? hist[w][e[r]] : 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (live && (m & below) == 0) hist[w][e[r]] = base + __popcll(m);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            rk[r] = base + __popcll(m & below);
+        }
+    __syncthreads();
+    // the experts' counts c and row blocks nb, scanned (ic, ib: inclusive, in the expert's wave, then over the 4 waves)
+    int c = 0, nb = 0, ic = 0, ib = 0;
+    if (t < 256)
+    {
+        #pragma unroll
+        for (int v = 0; v < DS_W; ++v) c += hist[v][t];
+        nb = t < n ? (c + bm - 1) / bm : 0;
+        ic = c; ib = nb;
+        #pragma unroll
+        for (int off = 1; off < 64; off <<= 1)
+        {
+            const int a = __shfl_up(ic, off), b = __shfl_up(ib, off);
+            if (l >= off) { ic += a; ib += b; }
+        }
+        if (l == 63) { wc[w] = ic; wb[w] = ib; }
+    }
+    __syncthreads();
+    if (t < 256)
+        for (int v = 0; v < w; ++v) { ic += wc[v]; ib += wb[v]; }
+    if (t < n)
+    {
+        int run = ic - c;
+        #pragma unroll
+        for (int v = 0; v < DS_W; ++v) { const int h = hist[v][t]; hist[v][t] = run; run += h; }
+        counts[t] = c;
+        disp_blocks(t, c, nb, bm, balance, ic - c, ib - nb, rbt, nrb_max);
+    }
+    if (t == 255) { meta[0] = ic; meta[1] = min(ib, nrb_max); meta[2] = ib; meta[3] = 0; }
+    __syncthreads();
+    #pragma unroll
+    for (int r = 0; r < DS_RND; ++r)
+    {
+        const int i = p0 + 64 * r + l;
+        if (r >= rounds || i >= F) continue;
+        if (e[r] < 0) { inv[i] = -1; continue; }
+        const int p = hist[w][e[r]] + rk[r];
+        tok[p] = i / topk; eid[p] = e[r]; wt[p] = (float) __builtin_bit_cast(_Float16, wv[r]); inv[i] = p;
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -516,6 +616,12 @@ extern "C" int hmoe_dispatch(const int64_t* sel, const uint16_t* rw, int T, int 
     int* hist = (int*) work;
     int* rank = hist + (size_t) nblk * n;
     hipStream_t st = (hipStream_t) stream;
+    if (F <= DS_PICKS)
+    {
+        disp_one_kernel<<<1, DS_W * 64, 0, st>>>(sel, rw, F, topk, lo, n, bm, balance, counts, tok, eid, wt, inv, rbt, nrb_max,
+                                                 meta);
+        return HMOE_LAUNCHED("dispatch");
+    }
     disp_count_kernel<<<nblk, DBLK, 0, st>>>(sel, F, lo, n, hist, rank);
     disp_scan_kernel<<<1, 1024, 0, st>>>(hist, nblk, n, bm, balance, counts, rbt, nrb_max, meta);
     disp_place_kernel<<<nblk, DBLK, 0, st>>>(sel, rw, F, topk, lo, n, hist, rank, tok, eid, wt, inv);
