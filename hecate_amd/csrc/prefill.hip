@@ -808,7 +808,24 @@ static int moe4t_run(const void* x, const int* tok, const float* wt, const int* 
         to_f16_kernel<<<TF16_GRID, 256, 0, st>>>((const uint16_t*) x, (size_t) T * H, (_Float16*) d);
         xh = (const _Float16*) d;
     }
-    if (nrb > 0)
+    // Which grouped GEMM, by the picks an expert has on average (npos counts those outside the window too, so for a partial
+    // window the line comes earlier). pgemm16_kernel runs a whole 256-pick block in one pass, but always stages, reads and
+    // loops for 16 tiles; pgemm.h's pass follows the block's tiles and takes a longer block as two. Gate/up + down, 256
+    // experts, us: 2100 tokens 1248 + 692 against 959 + 525, 3000: 1444 + 816 against 1193 + 667, 4096 (128 picks an expert):
+    // 1713 + 954 against 1659 + 923, 6000 (188): 2188 + 1249 against 2244 + 1250, 8192 (256): 3105 + 1726 against 3236 + 1792;
+    // whole layer 4300 tokens (134) 3615 against 3582, 4600 (144) 3766 against 3816.
+    if (nrb > 0 && npos <= 132 * n_tab)
+    {
+        PgArgs g{};
+        g.xin = xh; g.tok = tok; g.wt = wt; g.rbt = rbt; g.meta = meta;
+        g.w0 = gw; g.w1 = uw; g.s0 = gs; g.s1 = us; g.out = ar;
+        g.nrb = nrb; g.n_tab = n_tab; g.T = T; g.np = npos; g.ps = ps;
+        if (int rc = grouped_gate_up(g, EPI_ACT, st)) return rc;
+        g.xin = (const _Float16*) ar; g.w0 = dw; g.s0 = ds; g.w1 = g.s1 = nullptr;
+        g.out = inv ? (void*) d : (void*) out;
+        if (int rc = grouped_down(g, inv ? EPI_D16 : EPI_FIN, st)) return rc;
+    }
+    else if (nrb > 0)
     {
         // 256-pick blocks in one pass: 8 waves, each one 16-row strip of gate and of up (or two of down) against the
         // block's 16 pick tiles
