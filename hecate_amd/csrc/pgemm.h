@@ -10,7 +10,7 @@
 //     5 tiles; 2 above, where the accumulators need the registers); the row scales 4 groups at a time;
 //   * input rows: stages of 64 k by direct global-to-LDS loads into a ring of NBUF stages (8 up to 5 tiles, 4 above;
 //     80 KB, so that two workgroups share a CU), issued NBUF - 2 stages before they are read;
-//   * each 32-k step's input fragments are read from LDS one step ahead (WN tiles ahead above 6 tiles), each read issued
+//   * each 32-k step's input fragments are read from LDS one step ahead (WN tiles ahead above 5 tiles), each read issued
 //     behind the MFMAs that free its registers.
 // Every load is one the compiler sees (the stage ring is eight separate LDS arrays at compile-time indices, so that it
 // can tell a stage being filled from the one being read), so its waits count exactly and no wait drains the rings. The
@@ -246,9 +246,9 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
     const int ncb = NMAT == 2 ? 1 : ncb_;                   // (gate/up: one, which frees the rings for its epilogue)
     constexpr int K = NMAT == 2 ? H : I, NOUT = NMAT == 2 ? I : H, KG = K / 128, KS = K / 64, NS = 4 / NMAT;
     constexpr int NBUF = NT <= PG_STL ? 8 : 4;              // input stages in LDS
-    constexpr int WN = NT > 6 ? 2 : NT > 5 ? 3 : NT;        // input fragments held
+    constexpr int WN = NT == 8 ? 2 : NT == 7 ? 4 : NT == 6 ? 3 : NT;      // input fragments held
     constexpr int ND = (NT + 1) / 2;
-    static_assert(NT % WN == 0 && KS % 8 == 0 && (D == 2 || D == 4), "the loop is unrolled over 8 stages");
+    static_assert(WN <= NT && 16 * NT % WN == 0 && KS % 8 == 0 && (D == 2 || D == 4), "the loop is unrolled over 8 stages");
     const int t = threadIdx.x, l = t & 63, row = l & 15;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);   // wave index, kept in a scalar register
     const int nb0 = (cb0 * 4 + w) * NS;
@@ -359,11 +359,13 @@ __device__ __forceinline__ void pg_pass(BUF buf, const PgArgs& a, const Block& b
                 #pragma unroll
                 for (int i = 0; i < NT; ++i)
                 {
+                    // (fragments take the window's slots in turn, across the 16 steps of the unrolled loop)
+                    const int q = ((2 * s8 + k) * NT + i) % WN;
                     #pragma unroll
-                    for (int f = 0; f < 4; ++f) acc[f][i] = mfma16(aw[f], bq[i % WN], acc[f][i]);
+                    for (int f = 0; f < 4; ++f) acc[f][i] = mfma16(aw[f], bq[q], acc[f][i]);
                     // the fragment WN tiles on: of this step, or of the next one
-                    if (i + WN < NT) bq[i % WN] = rd(ic<J0>{}, i + WN, k);
-                    else bq[i % WN] = k == 0 ? rd(ic<J0>{}, i + WN - NT, 1) : rd(ic<J1>{}, i + WN - NT, 0);
+                    if (i + WN < NT) bq[q] = rd(ic<J0>{}, i + WN, k);
+                    else bq[q] = k == 0 ? rd(ic<J0>{}, i + WN - NT, 1) : rd(ic<J1>{}, i + WN - NT, 0);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             });
@@ -533,6 +535,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
             case 4: pg_pass<EPI, 4, 4>(buf, a, b, cbi * a.ncb, a.ncb); break;
             case 5: pg_pass<EPI, 5, 4>(buf, a, b, cbi * a.ncb, a.ncb); break;
             case 6: pg_pass<EPI, 6, 2>(buf, a, b, cbi * a.ncb, a.ncb); break;
+            case 7: pg_pass<EPI, 7, 2>(buf, a, b, cbi * a.ncb, a.ncb); break;
             default: pg_pass<EPI, 8, 2>(buf, a, b, cbi * a.ncb, a.ncb); break;
         }
     }
