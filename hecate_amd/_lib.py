@@ -44,11 +44,14 @@ SIGNATURES = {
                                       P, P, P, i32, P, P]),
     "hmoe_shared_work_bytes": (sz, [i32]),
     "hmoe_shared_forward": (i32, [P, i32, P, P, P, P, P, i32, P]),
+    "hmoe_shared_rows": (i32, [P, i32, P, P, P, P, P, i32, P]),
     "hmoe_moe4t_scratch_bytes": (sz, [i32, i32]),
     "hmoe_moe4t_forward": (i32, [P, P, P, P, P, i32, i32, i32, P, P, P, P, P, P, P, P, P, P, i32, P, i32, i32, P, i32,
                                  P]),
     "hmoe_moe4t_forward_bf16": (i32, [P, P, P, P, P, i32, i32, i32, P, P, P, P, P, P, P, P, P, P, i32, P, i32, i32, P,
                                       i32, P, P]),
+    "hmoe_moe4t_forward_base_bf16": (i32, [P, P, P, P, P, i32, i32, i32, P, P, P, P, P, P, P, P, P, P, i32, P, i32, i32,
+                                           P, i32, P, P]),
     "hmoe_moe4t_gemm": (i32, [P, i32, P, i32, i32, P, P, P, P, P, i32, i32, P]),
     "hmoe_residual_rmsnorm": (i32, [P, P, P, i32, f32, P, P, P]),
     "hmoe_combine_norm": (i32, [P, P, P, i32, P, P, P, P, P, f32, f32, f32, i32, i32, P]),

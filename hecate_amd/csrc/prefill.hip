@@ -534,8 +534,8 @@ __global__ void __launch_bounds__(256) to_f16_kernel(const uint16_t* __restrict_
 // select at its add), so all of them are in flight together: under a branch each load was followed by a wait for it.
 // MODE PF_ADD: out += the sum; PF_BF16: the sum goes to ob as bf16 (the partial out taken as zero and left untouched),
 // as PF_ADD into a zeroed out followed by finish_bf16 (0 + s is s, and s is never -0: it starts at +0); PF_FIN: ob =
-// bf16(out + sum) and out zeroed, as PF_ADD followed by finish_bf16
-enum { PF_ADD = 0, PF_BF16 = 1, PF_FIN = 2 };
+// bf16(out + sum) and out zeroed, as PF_ADD followed by finish_bf16; PF_BASE: as PF_FIN with out only read
+enum { PF_ADD = 0, PF_BF16 = 1, PF_FIN = 2, PF_BASE = 3 };
 template <int MODE>
 __global__ void __launch_bounds__(256) pfin_kernel(const _Float16* __restrict__ d, const int* __restrict__ inv, int topk,
                                                    int np, int sh_off, float* __restrict__ out, uint16_t* __restrict__ ob)
@@ -569,11 +569,11 @@ __global__ void __launch_bounds__(256) pfin_kernel(const _Float16* __restrict__ 
         }
         if constexpr (MODE != PF_ADD)
         {
-            if constexpr (MODE == PF_FIN)
+            if constexpr (MODE == PF_FIN || MODE == PF_BASE)
             {
                 f32x4* o = (f32x4*) (out + (size_t) t * H + n);
                 s = *o + s;
-                *o = (f32x4) {0.f, 0.f, 0.f, 0.f};
+                if constexpr (MODE == PF_FIN) *o = (f32x4) {0.f, 0.f, 0.f, 0.f};
             }
             uint32_t w[2];
             #pragma unroll
@@ -741,8 +741,8 @@ static size_t shw_end(int T) { return shw_act(T) + (((size_t) T * I * 2 + 255) &
 
 extern "C" size_t hmoe_shared_work_bytes(int T) { return shw_end(T > 0 ? T : 1); }
 
-extern "C" int hmoe_shared_forward(const void* x, int T, const void* sh_gw, const void* sh_uw, const void* sh_dw,
-                                   void* work, float* out, int xf, void* stream)
+static int shared_run(const void* x, int T, const void* sh_gw, const void* sh_uw, const void* sh_dw, void* work, float* out,
+                      int xf, bool add, void* stream)
 {
     if (T == 0) return HMOE_OK;
     HMOE_REQUIRE(x && sh_gw && sh_uw && sh_dw && work && out && T > 0, "shared_forward: arguments");
@@ -761,9 +761,21 @@ extern "C" int hmoe_shared_forward(const void* x, int T, const void* sh_gw, cons
     }
     _Float16* a = (_Float16*) (wk + shw_act(T));
     if (int rc = dense_gate_up((const _Float16*) sh_gw, (const _Float16*) sh_uw, xs, T, a, st)) return rc;
-    // (out += each product element once, in the GEMM's epilogue)
-    if (int rc = dense_down((const _Float16*) sh_dw, a, T, out, st)) return rc;
+    // (each product element added or written once, in the GEMM's epilogue)
+    if (int rc = dense_down((const _Float16*) sh_dw, a, T, out, add, st)) return rc;
     return HMOE_LAUNCHED("shared_forward");
+}
+
+extern "C" int hmoe_shared_forward(const void* x, int T, const void* sh_gw, const void* sh_uw, const void* sh_dw,
+                                   void* work, float* out, int xf, void* stream)
+{
+    return shared_run(x, T, sh_gw, sh_uw, sh_dw, work, out, xf, true, stream);
+}
+
+extern "C" int hmoe_shared_rows(const void* x, int T, const void* sh_gw, const void* sh_uw, const void* sh_dw, void* work,
+                                float* out, int xf, void* stream)
+{
+    return shared_run(x, T, sh_gw, sh_uw, sh_dw, work, out, xf, false, stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -781,15 +793,16 @@ extern "C" size_t hmoe_moe4t_scratch_bytes(int which, int npos)
     }
 }
 
-// moe4t forward; ob (with inv): the combine writes bf16(out + picks) to ob and zeroes out
+// moe4t forward; ob (with inv): the combine writes bf16(out + picks) to ob and zeroes out, or with base reads it (out is
+// the base, or NULL: none)
 static int moe4t_run(const void* x, const int* tok, const float* wt, const int* rbt, int npos, int nrb, int n_tab,
                      const int64_t* gw, const int64_t* uw, const int64_t* dw, const int64_t* gs, const int64_t* us,
                      const int64_t* ds, uint16_t* ar, float* d, float* out, int ps, const int* meta, int T, int xf,
-                     const int* inv, int topk, uint16_t* ob, void* stream)
+                     const int* inv, int topk, uint16_t* ob, bool base, void* stream)
 {
-    if (npos == 0) return HMOE_OK;                                      // moe4t.cu:508: no pick, no work
-    HMOE_REQUIRE(x && tok && wt && rbt && ar && out, "moe4t_forward: null buffer");
-    HMOE_REQUIRE(npos > 0 && nrb >= 0 && npos <= ps && T >= 1, "moe4t_forward: npos %d nrb %d ps %d T %d", npos, nrb, ps,
+    if (npos == 0 && !base) return HMOE_OK;                                      // moe4t.cu:508: no pick, no work
+    HMOE_REQUIRE(x && tok && wt && rbt && ar && (out || base), "moe4t_forward: null buffer");
+    HMOE_REQUIRE(npos >= 0 && nrb >= 0 && npos <= ps && T >= 1, "moe4t_forward: npos %d nrb %d ps %d T %d", npos, nrb, ps,
                  T);
     HMOE_REQUIRE((size_t) T * H * 2 <= UINT32_MAX && (size_t) ps * I * 2 <= UINT32_MAX,
                  "moe4t_forward: T %d ps %d past the 4 GB input offsets", T, ps);
@@ -839,7 +852,11 @@ static int moe4t_run(const void* x, const int* tok, const float* wt, const int* 
             pgemm16_kernel<1, 2, 4, EPI_FIN><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar, tok,
                 nullptr, rbt, nrb, meta, n_tab, dw, nullptr, ds, nullptr, nullptr, nullptr, T, 0, npos, out);
     }
-    if (inv && ob) pfin_kernel<PF_FIN><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, -1, out, ob);
+    // The base form neither zeroes the partial here nor reads it in the shared expert's down GEMM; both are HBM-bound on
+    // these rows (8192 tokens: 244 -> 220 us here, 280 -> 244 us there, rocprofv3 averages)
+    if (base && out) pfin_kernel<PF_BASE><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, -1, out, ob);
+    else if (base) pfin_kernel<PF_BF16><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, -1, nullptr, ob);
+    else if (inv && ob) pfin_kernel<PF_FIN><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, -1, out, ob);
     else if (inv) pfin_kernel<PF_ADD><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, -1, out, nullptr);
     return HMOE_LAUNCHED("moe4t_forward");
 }
@@ -852,7 +869,7 @@ extern "C" int hmoe_moe4t_forward(const void* x, const int* tok, const int* eid,
 {
     (void) eid; (void) gu;
     return moe4t_run(x, tok, wt, rbt, npos, nrb, n_tab, gw, uw, dw, gs, us, ds, ar, d, out, ps, meta, T, xf, inv, topk,
-                     nullptr, stream);
+                     nullptr, false, stream);
 }
 
 extern "C" int hmoe_moe4t_forward_bf16(const void* x, const int* tok, const int* eid, const float* wt, const int* rbt,
@@ -867,7 +884,20 @@ extern "C" int hmoe_moe4t_forward_bf16(const void* x, const int* tok, const int*
     // no pick: the output is the partial alone (finish_bf16 rounds it and zeroes it)
     if (npos == 0) return hmoe_finish_bf16(out, T, out_bf16, stream);
     return moe4t_run(x, tok, wt, rbt, npos, nrb, n_tab, gw, uw, dw, gs, us, ds, ar, d, out, ps, meta, T, xf, inv, topk,
-                     out_bf16, stream);
+                     out_bf16, false, stream);
+}
+
+extern "C" int hmoe_moe4t_forward_base_bf16(const void* x, const int* tok, const int* eid, const float* wt, const int* rbt,
+                                            int npos, int nrb, int n_tab, const int64_t* gw, const int64_t* uw,
+                                            const int64_t* dw, const int64_t* gs, const int64_t* us, const int64_t* ds,
+                                            float* gu, uint16_t* ar, float* d, const float* base, int ps, const int* meta,
+                                            int T, int xf, const int* inv, int topk, uint16_t* out_bf16, void* stream)
+{
+    (void) eid; (void) gu;
+    HMOE_REQUIRE(out_bf16 && inv && d && T >= 1 && ps >= 1 && ((uintptr_t) out_bf16 & 7) == 0,
+                 "moe4t_forward_base_bf16: needs d, the inverse map and an 8-byte aligned bf16 output");
+    return moe4t_run(x, tok, wt, rbt, npos, nrb, n_tab, gw, uw, dw, gs, us, ds, ar, d, (float*) base, ps, meta, T, xf, inv,
+                     topk, out_bf16, true, stream);
 }
 
 extern "C" int hmoe_moe4t_gemm(const void* xs, int rows, const int* rbt, int nrb, int n_tab, const int64_t* w0,

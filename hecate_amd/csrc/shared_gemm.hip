@@ -2,7 +2,7 @@
 // operands, fp32 accumulation); next to routed picks it rides in the grouped GEMM's launches instead (pgemm.h). The shared expert is a dense bf16 MLP (its weights are exact in f16), run over every token of the
 // chunk; the reference keeps it outside its routed op at prefill (runtime/tier/tier_split.py:548-560, the model's own
 // shared-expert forward). gate and up run as one GEMM whose epilogue writes act = f16(silu(g) u); down adds its rows into
-// fp32 out.
+// fp32 out or writes them.
 //
 // dgemm_kernel: D[n][m] = sum_k X[n][k] W[m][k] over row-major W [M][K] (one matrix, or gate and up as two) and X
 // [N][K]. Workgroup = WM x WN waves (WM along the weight rows, WN along the tokens) = 16 WM TM / NMAT output rows x
@@ -19,7 +19,7 @@
 
 namespace hmoe {
 
-enum { DG_ACT = 0, DG_ADD = 1 };
+enum { DG_ACT = 0, DG_ADD = 1, DG_SET = 2 };
 
 template <int NMAT, int TM, int TN, int WM, int WN, int EPI>
 __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WM * WN / 4, WM * WN / 4)))
@@ -157,7 +157,7 @@ dgemm_kernel(
             else
             {
                 f32x4* o = (f32x4*) ((float*) out + (size_t) n * ldo + m);
-                *o = *o + acc[i][j];
+                *o = EPI == DG_SET ? acc[i][j] : *o + acc[i][j];
             }
         }
     }
@@ -184,7 +184,7 @@ int hmoe::dense_gate_up(const _Float16* wg, const _Float16* wu, const _Float16* 
     return HMOE_LAUNCHED("shared gate/up");
 }
 
-int hmoe::dense_down(const _Float16* wd, const _Float16* act, int T, float* out, hipStream_t st)
+int hmoe::dense_down(const _Float16* wd, const _Float16* act, int T, float* out, bool add, hipStream_t st)
 {
     constexpr int BM = 16 * DN_WM * DN_TM, BN = 16 * DN_WN * DN_TN;
     static_assert(H % BM == 0 && I % 64 == 0, "down tiling");
@@ -192,6 +192,7 @@ int hmoe::dense_down(const _Float16* wd, const _Float16* act, int T, float* out,
                  "shared down: T %d or alignment", T);
     const dim3 g(H / BM, (T + BN - 1) / BN);
     constexpr int NT = 64 * DN_WM * DN_WN;
-    dgemm_kernel<1, DN_TM, DN_TN, DN_WM, DN_WN, DG_ADD><<<g, NT, 0, st>>>(wd, nullptr, act, T, I, out, H);
+    if (add) dgemm_kernel<1, DN_TM, DN_TN, DN_WM, DN_WN, DG_ADD><<<g, NT, 0, st>>>(wd, nullptr, act, T, I, out, H);
+    else dgemm_kernel<1, DN_TM, DN_TN, DN_WM, DN_WN, DG_SET><<<g, NT, 0, st>>>(wd, nullptr, act, T, I, out, H);
     return HMOE_LAUNCHED("shared down");
 }

@@ -23,17 +23,22 @@ def scratch(dev, npos):
 
 
 def forward(x, tok, eid, wt, rbt, gw, uw, dw, gs, us, ds, gu, ar, d, out, meta=None, npos=None, nrb=None, inv=None,
-            topk=8, out_bf16=None):
+            topk=8, out_bf16=None, base=None):
     """moe4t.cu:498-524: out[tok] += routed experts of the sorted picks; x fp16 (as the reference) or bf16 [T, H].
     inv (the dispatch's inverse map, this build's addition): each token adds its picks in top-k order (deterministic)
     instead of the down GEMM's atomic adds. out_bf16 (bf16 [T, H], with inv): the combine also rounds out to it and
-    zeroes out, as forward followed by moe4.finish_bf16 (hmoe_moe4t_forward_bf16)"""
-    on_device("moe4t", x, tok, eid, wt, rbt, gw, uw, dw, gs, us, ds, gu, ar, d, out, meta, inv)
+    zeroes out, as forward followed by moe4.finish_bf16 (hmoe_moe4t_forward_bf16). out None (with out_bf16): out_bf16 =
+    bf16(base + the picks), base fp32 [T, H] read only, or None (hmoe_moe4t_forward_base_bf16)"""
+    on_device("moe4t", x, tok, eid, wt, rbt, gw, uw, dw, gs, us, ds, gu, ar, d, out, meta, inv, base)
     T = x.shape[0]
-    if not (x.dim() == 2 and x.shape[1] == H and x.is_contiguous() and out.dtype == torch.float32
-            and out.is_contiguous() and out.shape[-1] == H and out.numel() >= T * H and rbt.dim() == 2
-            and rbt.shape[1] == 4 and rbt.dtype == torch.int32 and tok.dtype == torch.int32
-            and wt.dtype == torch.float32):
+    if out_bf16 is None and out is None or base is not None and out is not None:
+        raise RuntimeError("moe4t: the rows go to out, or to out_bf16 with base in out's place")
+    rows = base if out is None else out
+    if rows is not None and not (rows.dtype == torch.float32 and rows.is_contiguous() and rows.shape[-1] == H
+                                 and rows.numel() >= T * H):
+        raise RuntimeError("moe4t: shapes")
+    if not (x.dim() == 2 and x.shape[1] == H and x.is_contiguous() and rbt.dim() == 2 and rbt.shape[1] == 4
+            and rbt.dtype == torch.int32 and tok.dtype == torch.int32 and wt.dtype == torch.float32):
         raise RuntimeError("moe4t: shapes")
     npos = tok.numel() if npos is None else int(npos)
     nrb = rbt.shape[0] if nrb is None else int(nrb)
@@ -48,6 +53,11 @@ def forward(x, tok, eid, wt, rbt, gw, uw, dw, gs, us, ds, gu, ar, d, out, meta=N
                 or tuple(out_bf16.shape) != (T, H):
             raise RuntimeError("moe4t: out_bf16 (bf16 [T, H]) needs the inverse map")
         on_device("moe4t", out_bf16)
+        if out is None:
+            call("hmoe_moe4t_forward_base_bf16", ptr(x), ptr(tok), ptr(eid), ptr(wt), ptr(rbt), npos, nrb, gw.numel(),
+                 ptr(gw), ptr(uw), ptr(dw), ptr(gs), ptr(us), ptr(ds), ptr(gu), ptr(ar), ptr(d), ptr(base), ps,
+                 ptr(meta), T, xf_of(x), ptr(inv), int(topk), ptr(out_bf16), stream_of(x.device))
+            return
         call("hmoe_moe4t_forward_bf16", ptr(x), ptr(tok), ptr(eid), ptr(wt), ptr(rbt), npos, nrb, gw.numel(), ptr(gw),
              ptr(uw), ptr(dw), ptr(gs), ptr(us), ptr(ds), ptr(gu), ptr(ar), ptr(d), ptr(out), ps, ptr(meta), T,
              xf_of(x), ptr(inv), int(topk), ptr(out_bf16), stream_of(x.device))
@@ -74,13 +84,14 @@ def gemm(xs, rbt, w0, w1, out, down, s0=None, s1=None):
     return out
 
 
-def shared(x, sh_gw, sh_uw, sh_dw, work, out):
-    """the shared expert alone over a chunk (hmoe_shared_forward): out fp32 [T, H] += its SwiGLU MLP of x"""
+def shared(x, sh_gw, sh_uw, sh_dw, work, out, add=True):
+    """the shared expert alone over a chunk (hmoe_shared_forward): out fp32 [T, H] += its SwiGLU MLP of x (add False:
+    the rows written, out not read: hmoe_shared_rows)"""
     on_device("shared", x, sh_gw, sh_uw, sh_dw, work, out)
     T = x.shape[0]
     if work.numel() * work.element_size() < int(lib().hmoe_shared_work_bytes(T)):
         raise RuntimeError("shared: work too small")
     if not all(w.dtype == torch.float16 and w.is_contiguous() and w.numel() == I * H for w in (sh_gw, sh_uw, sh_dw)):
         raise RuntimeError("shared: weights are row-major f16 gate [I, H], up [I, H], down [H, I]")
-    call("hmoe_shared_forward", ptr(x), T, ptr(sh_gw), ptr(sh_uw), ptr(sh_dw), ptr(work), ptr(out), xf_of(x),
-         stream_of(x.device))
+    call("hmoe_shared_forward" if add else "hmoe_shared_rows", ptr(x), T, ptr(sh_gw), ptr(sh_uw), ptr(sh_dw), ptr(work),
+         ptr(out), xf_of(x), stream_of(x.device))

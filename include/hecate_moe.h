@@ -220,6 +220,14 @@ int hmoe_moe4t_forward_bf16(const void* x, const int* tok, const int* eid, const
                             const int64_t* gs, const int64_t* us, const int64_t* ds, float* gu, uint16_t* ar, float* d,
                             float* out, int ps, const int* meta, int T, int xf, const int* inv, int topk,
                             uint16_t* out_bf16, void* stream);
+/* The same with a partial that is only read: out_bf16 = bf16(base + picks), base fp32 [T][H] or NULL (no partial). For the
+ * layer's long prefill, the shared expert's rows from hmoe_shared_rows as the base: no fp32 buffer has to be kept
+ * zeroed. d and inv are required; npos = 0 gives the base alone. */
+int hmoe_moe4t_forward_base_bf16(const void* x, const int* tok, const int* eid, const float* wt, const int* rbt, int npos,
+                                 int nrb, int n_tab, const int64_t* gw, const int64_t* uw, const int64_t* dw,
+                                 const int64_t* gs, const int64_t* us, const int64_t* ds, float* gu, uint16_t* ar,
+                                 float* d, const float* base, int ps, const int* meta, int T, int xf, const int* inv,
+                                 int topk, uint16_t* out_bf16, void* stream);
 /* runtime/tier/moe4/moe4t.cu:476-488 moe4t_gemm(xs, rbt, w0, w1, out, down), the test entry: one grouped GEMM over
  * row blocks of <= 256 picks whose inputs are rows p of xs f16 [rows][K]. Gate/up shape (down = 0, K = H): out fp32
  * [2][ps][I] = the gate (w0, s0) and up (w1, s1) sums; down shape (down = 1, K = I): out fp32 [ps][H] (w0, s0). The
@@ -236,6 +244,9 @@ int hmoe_moe4t_gemm(const void* xs, int rows, const int* rbt, int nrb, int n_tab
 size_t hmoe_shared_work_bytes(int T);
 int hmoe_shared_forward(const void* x, int T, const void* sh_gw, const void* sh_uw, const void* sh_dw, void* work,
                         float* out, int xf, void* stream);
+/* the same rows written: out = down(silu(gate x) * up x), out not read */
+int hmoe_shared_rows(const void* x, int T, const void* sh_gw, const void* sh_uw, const void* sh_dw, void* work, float* out,
+                     int xf, void* stream);
 
 /* ---- residual + RMSNorm: runtime/tier/cn.cu and runtime/core/nr4_kernel.cuh ----
  * Every RMSNorm here uses the reduction order of the reference's rms_norm_kernel, which its fused kernels reproduce

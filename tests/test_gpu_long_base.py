@@ -1,0 +1,51 @@
+"""The long prefill's combine over a partial that is only read (moe4t.forward with base in out's place) and the shared
+expert's rows written instead of added: bit for bit the forms that add into a zeroed fp32 partial and re-zero it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+H = 6144
+
+
+@pytest.fixture(scope="module")
+def lay():
+    from hecate_amd import synth
+    return synth.make_layer(0, torch.device("cuda:0"), resident=[3, 7])
+
+
+@pytest.mark.parametrize("picks", (True, False))
+@pytest.mark.parametrize("T", (1, 127, 129, 700))
+def test_base_rows(lay, T, picks):
+    from hecate_amd import _lib, moe4t, synth, tier
+    dev = lay.device
+    x = synth.gen_x(900 + T, T, dev).half()
+    sel = torch.full((T, 2), 2, dtype=torch.int64, device=dev)           # outside the window
+    if picks:
+        sel[:, 0] = torch.arange(T, device=dev) % 3                      # experts 0 and 1, and every third token neither
+    rw = torch.full((T, 2), 0.5, dtype=torch.float16, device=dev)
+    pf = tier.PrefillBuffers(T, 2, 0, 2, 256, dev, bm=256, long=True).run(sel, rw)
+    gq, uq, dq, gs, us, ds = lay.bank.tables()
+    a = (x, pf.tok, pf.eid, pf.wt, pf.rbt, gq, uq, dq, gs, us, ds, *pf.scr)
+    kw = dict(meta=pf.meta, npos=pf.F, nrb=pf.nrb_max, inv=pf.inv, topk=2)
+    y = torch.zeros((T, H), device=dev)
+    moe4t.shared(x, *lay.shared_rows(), pf.shw, y)
+    sh = torch.full((T, H), float("nan"), device=dev)
+    moe4t.shared(x, *lay.shared_rows(), pf.shw, sh, add=False)
+    assert torch.equal(sh, y)
+    o = [torch.full((T, H), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(4)]
+    moe4t.forward(*a, None, out_bf16=o[0], base=sh, **kw)
+    assert torch.equal(sh, y)                                            # the base is read only
+    moe4t.forward(*a, y, out_bf16=o[1], **kw)
+    moe4t.forward(*a, None, out_bf16=o[2], **kw)                         # no base
+    moe4t.forward(*a, y, out_bf16=o[3], **kw)                            # (y zeroed by the call before)
+    assert torch.equal(o[0].view(torch.int16), o[1].view(torch.int16))
+    assert torch.equal(o[2].view(torch.int16), o[3].view(torch.int16))
+    kw["npos"] = 0                                                       # no pick: the base alone
+    moe4t.forward(*a, None, out_bf16=o[0], base=sh, **kw)
+    assert torch.equal(o[0], sh.bfloat16())
+    with pytest.raises(RuntimeError):
+        moe4t.forward(*a, y, out_bf16=o[0], base=sh, **kw)
+    with pytest.raises(RuntimeError):
+        moe4t.forward(*a, None, **kw)
+    assert _lib.lib().hmoe_moe4t_forward_base_bf16(*([None] * 5), 0, 0, 0, *([None] * 10), 0, None, 1, 0, None, 8, None,
+                                                   None) != 0
