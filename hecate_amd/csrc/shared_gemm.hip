@@ -1,7 +1,7 @@
 // shared_gemm.hip - the shared expert over a chunk by itself (hmoe_shared_forward) as hand-written dense MFMA GEMMs (f16
-// operands, fp32 accumulation); next to routed picks it rides in the grouped GEMM's launches instead (pgemm.h). The shared expert is a dense bf16 MLP (its weights are exact in f16), run over every token of the
-// chunk; the reference keeps it outside its routed op at prefill (runtime/tier/tier_split.py:548-560, the model's own
-// shared-expert forward). gate and up run as one GEMM whose epilogue writes act = f16(silu(g) u); down adds its rows into
+// operands, fp32 accumulation); up to 2048 tokens it rides in the grouped GEMM's launches instead (pgemm.h). The shared
+// expert is a dense bf16 MLP (its weights are exact in f16), run over every token of the chunk; the reference keeps it
+// outside its routed op at prefill (runtime/tier/tier_split.py:548-560, the model's own shared-expert forward). gate and up run as one GEMM whose epilogue writes act = f16(silu(g) u); down adds its rows into
 // fp32 out or writes them.
 //
 // dgemm_kernel: D[n][m] = sum_k X[n][k] W[m][k] over row-major W [M][K] (one matrix, or gate and up as two) and X
