@@ -88,7 +88,7 @@ struct PgArgs
     const int64_t* s1;
     void* out;
     int nrb, n_tab, T, np, ps;
-    int ncb;                                // column blocks per workgroup (set by the launchers)
+    int ncb, shb;                           // column blocks per workgroup: routed, shared (set by the launchers)
     // the shared expert (row-major f16 [N][K], NULL: none) on every one of the T tokens in the same launch: its rows follow
     // the picks' (row ps + t of the act, and of down's rows)
     const _Float16* sh0;
@@ -498,20 +498,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     if constexpr (EPI == EPI_ACT || EPI == EPI_D16)
     {
         // the shared expert's blocks come first: they are the longest, and the rest fills in around them. The token blocks of
-        // one column block go to consecutive workgroups of one XCD, which then reads its weights once.
-        const int ns = a.nsh * ny;
+        // one column block go to consecutive workgroups of one XCD, which then reads its weights once (NCB / shb is a
+        // multiple of 8: 16 in gate/up, 24 or 8 in down).
+        const int ns = a.nsh * (NCB / a.shb);
         if (i < ns)
         {
             const int j = i >> 3;
-            const int cb = (ny & 7) == 0 ? (j / a.nsh) * 8 + (i & 7) : i / a.nsh;
-            const int t0 = ((ny & 7) == 0 ? j : i) % a.nsh * a.sh_rows, rows = min(a.sh_rows, a.T - t0);
+            const int cb = (j / a.nsh) * 8 + (i & 7), t0 = j % a.nsh * a.sh_rows, rows = min(a.sh_rows, a.T - t0);
             if (rows <= 0) return;
             switch ((rows + 31) >> 5)
             {
-                case 1: pg_dense<EPI, 2, 4>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
-                case 2: pg_dense<EPI, 4, 4>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
-                case 3: pg_dense<EPI, 6, 2>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
-                default: pg_dense<EPI, 8, 2>(buf, a, t0, rows, cb * a.ncb, a.ncb); break;
+                case 1: pg_dense<EPI, 2, 4>(buf, a, t0, rows, cb * a.shb, a.shb); break;
+                case 2: pg_dense<EPI, 4, 4>(buf, a, t0, rows, cb * a.shb, a.shb); break;
+                case 3: pg_dense<EPI, 6, 2>(buf, a, t0, rows, cb * a.shb, a.shb); break;
+                default: pg_dense<EPI, 8, 2>(buf, a, t0, rows, cb * a.shb, a.shb); break;
             }
             return;
         }

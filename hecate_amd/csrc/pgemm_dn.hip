@@ -5,14 +5,22 @@ using namespace hmoe;
 
 int hmoe::grouped_down(const PgArgs& a, int epi, hipStream_t st)
 {
-    // A workgroup runs 3 column blocks in one pipeline: down's k loop is 16 groups, so with one column block a third of a
-    // workgroup's life is its prologue (150 tokens, 250 experts: 310 us with one, 287 with three). With few picks the
-    // launch is a few workgroups per CU and the shorter ones of 2 spread better (17 tokens, 103 experts: 123 against
-    // 133 us; equal at about 25 tokens).
+    // Column blocks per workgroup (times are whole moe4p.forward calls, us).
+    // Routed: three in one pipeline, since down's k loop is 16 groups and with one column block a third of a workgroup's
+    // life is its prologue (256 experts: 150 tokens 843 with one, 823 with three; 1000 tokens 1128, 1108). One where that
+    // leaves CUs without a workgroup, which then run three times as long: tables of few experts (8 experts: 450 tokens 71
+    // with one, 94 with three; 2048 tokens 116, 154; 48 experts: 187, 192 and 325, 332; from 64 on three again: 244, 237 and
+    // 415, 414), or few picks (17 tokens: 96 experts 159, 167; 256 experts 365, 364). Beside the shared expert's blocks the
+    // routed ones spread over fewer free slots, and the line is higher (33 tokens: 64 experts 226, 241; 450: 279, 293 and 96
+    // experts 400, 409; 128 experts 520, 518).
+    // Shared: one, its serial chain over k being the launch's length beside few experts (33 tokens, 8 experts 145 with one,
+    // 204 with three; 450 tokens, 32 experts 230, 290; 1000 tokens, 256 experts 1224, 1223). (The kernel takes the count at
+    // run time: with a constant one it spills two registers.)
     PgArgs g = a;
-    g.ncb = a.np < 200 ? 2 : 3;
+    g.ncb = a.np < 200 || a.n_tab < (a.sh0 ? 128 : 64) ? 1 : 3;
+    g.shb = 1;
     pg_shared_blocks(g);
-    const dim3 grid(pgemm_grid(a.nrb, H / 256 / g.ncb).x + g.nsh * (H / 256 / g.ncb));
+    const dim3 grid(pgemm_grid(a.nrb, H / 256 / g.ncb).x + g.nsh * (H / 256 / g.shb));
     if (grid.x == 0) return HMOE_OK;
     if (epi == EPI_D16) pgemm_kernel<EPI_D16><<<grid, 256, 0, st>>>(g);
     else if (epi == EPI_FIN) pgemm_kernel<EPI_FIN><<<grid, 256, 0, st>>>(g);

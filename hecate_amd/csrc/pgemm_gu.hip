@@ -6,7 +6,7 @@ using namespace hmoe;
 int hmoe::grouped_gate_up(const PgArgs& a, int epi, hipStream_t st)
 {
     PgArgs g = a;
-    g.ncb = 1;
+    g.ncb = g.shb = 1;
     pg_shared_blocks(g);
     const dim3 grid(pgemm_grid(a.nrb, I / 128).x + g.nsh * (I / 128));
     if (grid.x == 0) return HMOE_OK;
