@@ -35,9 +35,10 @@ __host__ __device__ __forceinline__ size_t sc_index(int n, int g, int KG)
 // ---- error state of the C ABI (common.hip) ----
 int set_error(int code, const char* fmt, ...);
 // the shared expert over a chunk (shared_gemm.hip), f16 row-major operands: act [T][I] = f16(silu(wg x) (wu x)), and
-// out [T][H] (fp32) += (add) or = wd act
+// wd act as out [T][H]: f16 rows (DG_MODE_F16), fp32 added (DG_MODE_ADD) or written (DG_MODE_SET)
 int dense_gate_up(const _Float16* wg, const _Float16* wu, const _Float16* x, int T, _Float16* act, hipStream_t st);
-int dense_down(const _Float16* wd, const _Float16* act, int T, float* out, bool add, hipStream_t st);
+enum { DG_MODE_F16 = 0, DG_MODE_ADD = 1, DG_MODE_SET = 2 };
+int dense_down(const _Float16* wd, const _Float16* act, int T, void* out, int mode, hipStream_t st);
 int hip_check(hipError_t e, const char* what);
 // the router's select launch for R <= MAXR rows of finished logits [R][RMAXE] (router.hip): one wave per row
 int router_select_small(const float* logits, const float* bias, int R, int E, int topk, float scale, int64_t* sel,

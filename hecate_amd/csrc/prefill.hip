@@ -685,18 +685,30 @@ static int moe4p_run(const void* x, const int* tok, const float* wt, const int* 
     // gate/up, then down into d rows for the ordered combine (inv given) or added into out[tok] by its epilogue (no
     // inverse map: the atomic combine of p4_fin_kernel)
     // The shared expert (every token) rides in the same two launches: act rows ps.. = f16(silu(gate x) up x), then down
-    // into d rows ps.. (f16), which the ordered combine adds after each token's picks
-    const bool sh = sh_gw != nullptr;
+    // into d rows ps.. (f16), which the ordered combine adds after each token's picks. Past 4096 tokens it takes the
+    // dense launches instead, whose larger tiles are the faster once there are enough of them (us, riding against apart:
+    // 8192 tokens, 8 experts 1040, 959, 256 experts 5711, 5616; 6000 tokens 750, 701 and 4303, 4246; 4096 tokens 562, 558 and
+    // 3126, 3193; 3000 tokens, 8 experts 381, 458).
+    const bool sh = sh_gw != nullptr, apart = sh && T > 4096;
     PgArgs g{};
     g.xin = (const _Float16*) xb; g.tok = tok; g.wt = wt; g.rbt = rbt; g.meta = meta;
     g.w0 = gw; g.w1 = uw; g.s0 = gs; g.s1 = us; g.out = a;
     g.nrb = nrb; g.n_tab = n_tab; g.T = T; g.np = npos; g.ps = ps;
-    g.sh0 = (const _Float16*) sh_gw; g.sh1 = (const _Float16*) sh_uw;
+    if (sh && !apart) { g.sh0 = (const _Float16*) sh_gw; g.sh1 = (const _Float16*) sh_uw; }
     if (int rc = grouped_gate_up(g, EPI_ACT, st)) return rc;
     g.xin = a; g.w0 = dw; g.s0 = ds; g.w1 = g.s1 = nullptr;
-    g.sh0 = (const _Float16*) sh_dw; g.sh1 = nullptr;
+    if (g.sh0) { g.sh0 = (const _Float16*) sh_dw; g.sh1 = nullptr; }
     g.out = inv ? d : out;
     if (int rc = grouped_down(g, inv ? EPI_D16 : EPI_FIN, st)) return rc;
+    if (apart)
+    {
+        if (int rc = dense_gate_up((const _Float16*) sh_gw, (const _Float16*) sh_uw, (const _Float16*) xb, T,
+                                   a + (size_t) ps * I, st))
+            return rc;
+        if (int rc = dense_down((const _Float16*) sh_dw, a + (size_t) ps * I, T, (_Float16*) d + (size_t) ps * H,
+                                DG_MODE_F16, st))
+            return rc;
+    }
     if (inv && ob) pfin_kernel<PF_BF16><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, sh ? ps : -1, nullptr, ob);
     else if (inv) pfin_kernel<PF_ADD><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, npos, sh ? ps : -1, out, nullptr);
     return HMOE_LAUNCHED("moe4p_forward");
@@ -762,7 +774,7 @@ static int shared_run(const void* x, int T, const void* sh_gw, const void* sh_uw
     _Float16* a = (_Float16*) (wk + shw_act(T));
     if (int rc = dense_gate_up((const _Float16*) sh_gw, (const _Float16*) sh_uw, xs, T, a, st)) return rc;
     // (each product element added or written once, in the GEMM's epilogue)
-    if (int rc = dense_down((const _Float16*) sh_dw, a, T, out, add, st)) return rc;
+    if (int rc = dense_down((const _Float16*) sh_dw, a, T, out, add ? DG_MODE_ADD : DG_MODE_SET, st)) return rc;
     return HMOE_LAUNCHED("shared_forward");
 }
 
