@@ -242,6 +242,11 @@ class PrefillBuffers:
         self.sel, self.rw = z(T, topk, dt=torch.int64), z(T, topk, dt=torch.float16)
         self.logits = z(int(L.hmoe_router_scratch_bytes(T, E)) // 4, dt=torch.float32)
 
+    def bounds(self, T):
+        """(picks, row blocks) a chunk of T rows can reach at most: what its plan's consumers are given. Not the buffers' own
+        capacity: the operators choose their kernels by these numbers, and the buffers may be of an earlier, larger chunk"""
+        return T * self.topk, int(lib().hmoe_dispatch_nrb_max(T * self.topk, self.n, self.bm))
+
     def run(self, sel, rw, balance=True):
         """device dispatch plan of a selection (tier_split.py:404-417 + pick_groups in one group), no host sync:
         counts, tok / eid / wt sorted by (expert, flat index), inv, rbt rows, meta = {npos, nrb, nrb wanted, 0}"""
@@ -340,6 +345,7 @@ class MoELayer:
         combine touches it. Returns whether out_bf16 was written (the atomic moe4t form adds into y instead)."""
         T = x.shape[0]
         pf = self._pf
+        npos, nrb = pf.bounds(T)
         gq, uq, dq, gs, us, ds = self.bank.tables()
         if pf.long:
             # tier_split.py:427-462: every routed expert on moe4t (256-pick balanced blocks, the down GEMM adding into
@@ -353,7 +359,7 @@ class MoELayer:
                 sh = pf.sh[:T]
                 moe4t.shared(x, *self.shared_rows(), pf.shw, sh, add=False)
             moe4t.forward(x, pf.tok, pf.eid, pf.wt, pf.rbt, gq, uq, dq, gs, us, ds, *pf.scr, None if fused else y,
-                          base=sh, meta=pf.meta, npos=pf.F, nrb=pf.nrb_max,
+                          base=sh, meta=pf.meta, npos=npos, nrb=nrb,
                           inv=pf.inv[:T * self.topk] if self.deterministic else None, topk=self.topk,
                           out_bf16=out_bf16 if fused else None)
             if not fused and with_shared and self.shared is not None:
@@ -362,7 +368,7 @@ class MoELayer:
         sh = self.shared_rows() if (with_shared and self.shared is not None) else None
         moe4p.forward(x, pf.tok, pf.eid, pf.wt, pf.rbt, gq, uq, dq, gs, us, ds, *pf.scr,
                       y if out_bf16 is None else None, inv=pf.inv[:T * self.topk], meta=pf.meta, topk=self.topk,
-                      shared=sh, npos=pf.F, nrb=pf.nrb_max, out_bf16=out_bf16)
+                      shared=sh, npos=npos, nrb=nrb, out_bf16=out_bf16)
         return out_bf16 is not None
 
     def shared_rows(self):

@@ -1,0 +1,42 @@
+"""The sizes a prefill chunk hands to its operators: the chunk's own, whatever chunk the layer's buffers were made for (the
+operators choose their kernels by them)."""
+import pytest
+import torch
+
+from hecate_amd import moe4p, moe4t, tier
+
+
+def _layer(E=16, n=2):
+    return tier.MoELayer(torch.zeros(E, 6144), torch.zeros(E), tier.ExpertBank(n, "cpu"), max_rows=16)
+
+
+@pytest.mark.parametrize("long,first,then", [(False, 300, 17), (False, 40, 40), (True, 300, 21)])
+def test_prefill_bounds(monkeypatch, long, first, then):
+    monkeypatch.setattr(tier, "LONG_ROWS", 16 if long else 2048)
+    lay, calls = _layer(), []
+    for mod in (moe4p, moe4t):
+        monkeypatch.setattr(mod, "forward", lambda *a, **k: calls.append(k))
+    for T in (first, then):
+        pf = lay._prefill_buffers(T)
+        assert pf.T == first and pf.long == long
+        lay.prefill_experts(pf.xh[:T], pf.y[:T])
+        bm = 256 if long else 128
+        assert calls[-1]["npos"] == T * 8 and calls[-1]["nrb"] == 2 + T * 8 // bm
+        assert calls[-1]["inv"].numel() == T * 8
+    assert len(calls) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("first,then", [(300, 17), (300, 40), (2300, 2100)])
+def test_prefill_after_a_larger_chunk(dev, first, then):
+    """a chunk after a larger one on the same layer: the bits of the same chunk on fresh buffers"""
+    from hecate_amd import synth
+    lay = synth.make_layer(0, dev, resident=[3, 7], max_rows=16)
+    x = synth.gen_x(31, first, dev)
+    fresh = lay.prefill(x[:then]).clone()
+    lay._pf = None
+    lay.prefill(x)
+    assert lay._pf.T == first
+    after = lay.prefill(x[:then])
+    assert lay._pf.T == first and bool(fresh.any())
+    assert torch.equal(after.view(torch.int16), fresh.view(torch.int16))
