@@ -233,14 +233,32 @@ class PrefillBuffers:
             self.scr = [None, torch.empty((F, I), dtype=torch.float16, device=dev),
                         torch.empty((F, H), dtype=torch.float16, device=dev)]
             self.shw = torch.empty(int(L.hmoe_shared_work_bytes(T)) // 4 + 64, dtype=torch.float32, device=dev)
-            self.sh = torch.empty((T, H), dtype=torch.float32, device=dev)      # the shared expert's rows
         else:
             self.scr = moe4p.scratch(dev, F, T)
-        self.y = z(T, H, dt=torch.float32)
+        self._y = self._sh = None
         self.out = z(T, H, dt=torch.bfloat16)
         self.xh = z(T, H, dt=torch.float16)                        # the router's f16 copy of x (the GEMM input)
         self.sel, self.rw = z(T, topk, dt=torch.int64), z(T, topk, dt=torch.float16)
         self.logits = z(int(L.hmoe_router_scratch_bytes(T, E)) // 4, dt=torch.float32)
+
+    # The two fp32 [T, H] buffers are made on first use: a layer needs at most one of them (the long prefill with the ordered
+    # combine sh, if it has a shared expert; with the atomic one y; the short prefill neither), 201 MB at 8192 rows
+    @property
+    def y(self):
+        """fp32 accumulator [T, H], kept zeroed"""
+        if self._y is None:
+            y = torch.zeros((self.T, H), dtype=torch.float32, device=self.out.device)
+            if y.is_cuda and torch.cuda.is_current_stream_capturing():
+                return y                                                # (zeros only once the graph runs: the graph's own)
+            self._y = y
+        return self._y
+
+    @property
+    def sh(self):
+        """the shared expert's rows [T, H] of the long prefill's ordered combine"""
+        if self._sh is None:
+            self._sh = torch.empty((self.T, H), dtype=torch.float32, device=self.out.device)
+        return self._sh
 
     def bounds(self, T):
         """(picks, row blocks) a chunk of T rows can reach at most: what its plan's consumers are given. Not the buffers' own
@@ -340,9 +358,9 @@ class MoELayer:
 
     def prefill_experts(self, x, y, with_shared=True, out_bf16=None):
         """routed (+ shared) experts of x's routed selection (in the prefill buffers) added into y fp32 [T, H].
-        With out_bf16 (bf16 [T, H]) the layer output bf16(experts) is written there instead, and y must hold zeros on
-        entry (as MoELayer keeps it) and holds zeros on return: neither the moe4p form nor the moe4t form with the ordered
-        combine touches it. Returns whether out_bf16 was written (the atomic moe4t form adds into y instead)."""
+        With out_bf16 (bf16 [T, H]) the layer output bf16(experts) is written there instead, and y is not touched: by
+        the moe4p form and the moe4t form with the ordered combine (y may be None for them). Returns whether out_bf16 was
+        written (the atomic moe4t form adds into y instead, which must hold zeros on entry)."""
         T = x.shape[0]
         pf = self._pf
         npos, nrb = pf.bounds(T)
@@ -394,8 +412,8 @@ class MoELayer:
         sel, rw = pf.sel[:T], pf.rw[:T]
         router.router_fused(x, self.wg, self.bias, pf.logits, self.ctr, sel, rw, self.topk, self.scale, pf.xh[:T])
         pf.run(sel, rw, balance=True)
-        y = pf.y[:T]
-        # (y is kept zeroed, so the moe4p path writes the bf16 output from its combine directly)
+        # (only the atomic combine needs the accumulator: the others write the bf16 output themselves)
+        y = pf.y[:T] if pf.long and not self.deterministic else None
         if self.prefill_experts(pf.xh[:T], y, with_shared, out_bf16=pf.out[:T]):
             return pf.out[:T]
         return moe4.finish_bf16(y, T, pf.out[:T])
