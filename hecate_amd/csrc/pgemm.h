@@ -41,8 +41,6 @@ struct Block { int e, p0, rows; };
 // XCDs (workgroup i runs on XCD i % 8), each with its own L2: the column blocks of one row block go to consecutive
 // workgroups of one XCD, so they run together and read the block's input rows from that XCD's L2 (one fetch from
 // memory instead of one per column block). i: the workgroup's index among nrb (rounded up to 8) x ny.
-// (the extents come from the launch's own arguments: gridDim reads the dispatch packet, a round trip to the queue's
-// memory at every workgroup start)
 __device__ __forceinline__ void xcd_tile(int i, int& rb, int& cb, int ny)
 {
     const int j = i >> 3;
@@ -50,7 +48,12 @@ __device__ __forceinline__ void xcd_tile(int i, int& rb, int& cb, int ny)
     cb = j % ny;
 }
 
-inline dim3 pgemm_grid(int nrb, int ny) { return dim3(((nrb + 7) & ~7) * ny); }
+// The grid of nrb row blocks x ny column blocks and extra x ny workgroups more, and a workgroup's index in it. Two
+// dimensions: a launch's x extent is at most 2^32 threads, which a plan of 524,288 blocks would pass in one. (x the extent
+// from the launch's own arguments: gridDim reads the dispatch packet, a round trip to the queue's memory at every workgroup
+// start)
+inline dim3 pgemm_grid(int nrb, int ny, int extra = 0) { return dim3(((nrb + 7) & ~7) + extra, ny); }
+__device__ __forceinline__ int pgemm_index(int gx) { return blockIdx.x + gx * blockIdx.y; }
 
 // a scalar load from memory that no kernel of the launch writes: under the weight stream a vector load returns behind
 // every load the CU has in flight (over 1 us), a scalar load does not wait for them. The address must be the same in
@@ -94,6 +97,7 @@ struct PgArgs
     const _Float16* sh0;
     const _Float16* sh1;
     int nsh, sh_rows;                       // its token blocks and the tokens of each (set by the launchers)
+    int gx;                                 // the grid's x extent (set by the launchers)
 };
 // the shared expert's token blocks: of equal size, whole tiles, at most PG_PB
 inline void pg_shared_blocks(PgArgs& a)
@@ -494,7 +498,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     constexpr int NMAT = EPI == EPI_ACT || EPI == EPI_RAW ? 2 : 1;
     constexpr int NCB = (NMAT == 2 ? I : H) / (256 / NMAT);
     const int ny = NCB / a.ncb;
-    int i = blockIdx.x;
+    int i = pgemm_index(a.gx);
     if constexpr (EPI == EPI_ACT || EPI == EPI_D16)
     {
         // the shared expert's blocks come first: they are the longest, and the rest fills in around them. The token blocks of

@@ -20,8 +20,9 @@ int hmoe::grouped_down(const PgArgs& a, int epi, hipStream_t st)
     g.ncb = a.np < 200 || a.n_tab < (a.sh0 ? 128 : 64) ? 1 : 3;
     g.shb = 1;
     pg_shared_blocks(g);
-    const dim3 grid(pgemm_grid(a.nrb, H / 256 / g.ncb).x + g.nsh * (H / 256 / g.shb));
+    const dim3 grid = pgemm_grid(a.nrb, H / 256 / g.ncb, g.nsh * g.ncb / g.shb);
     if (grid.x == 0) return HMOE_OK;
+    g.gx = grid.x;
     if (epi == EPI_D16) pgemm_kernel<EPI_D16><<<grid, 256, 0, st>>>(g);
     else if (epi == EPI_FIN) pgemm_kernel<EPI_FIN><<<grid, 256, 0, st>>>(g);
     else pgemm_kernel<EPI_D><<<grid, 256, 0, st>>>(g);

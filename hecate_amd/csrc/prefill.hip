@@ -271,7 +271,7 @@ __global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2
     __shared__ __attribute__((aligned(16))) u32x4 xs0[NTT * 4 * 64];
     __shared__ __attribute__((aligned(16))) u32x4 xs1[NTT * 4 * 64];
     int rbi, cbi;
-    xcd_tile(blockIdx.x, rbi, cbi, NOUT / (16 * NS * NWV));
+    xcd_tile(pgemm_index((nrb + 7) & ~7), rbi, cbi, NOUT / (16 * NS * NWV));
     Block rb;
     if (!get_block(rbt, nrb, meta, n_tab, np, rbi, rb)) return;
     // a block of more than PBX picks runs as passes of PBX, one after the other (a later pass reads the weights

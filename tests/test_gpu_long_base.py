@@ -49,3 +49,25 @@ def test_base_rows(lay, T, picks):
         moe4t.forward(*a, None, **kw)
     assert _lib.lib().hmoe_moe4t_forward_base_bf16(*([None] * 5), 0, 0, 0, *([None] * 10), 0, None, 1, 0, None, 8, None,
                                                    None) != 0
+
+
+@pytest.mark.parametrize("npos", (260, 600))
+def test_many_row_blocks(lay, npos):
+    """a plan's room for row blocks far past the plan (600,000, as blocks of one pick would need; the device's count says
+    how many there are), on either grouped GEMM: the bits of the same call with the plan's own room"""
+    from hecate_amd import moe4t, synth, tier
+    dev = lay.device
+    T = 130
+    x = synth.gen_x(70, T, dev).half()
+    sel = (torch.arange(2 * T, device=dev) % 3).view(T, 2)
+    rw = torch.full((T, 2), 0.5, dtype=torch.float16, device=dev)
+    pf = tier.PrefillBuffers(300, 2, 0, 2, 256, dev, bm=256, long=True).run(sel, rw)
+    rbt = torch.zeros((600000, 4), dtype=torch.int32, device=dev)
+    rbt[:pf.nrb_max] = pf.rbt
+    ys = []
+    for plan in (pf.rbt, rbt):
+        y = torch.zeros((T, H), device=dev)
+        moe4t.forward(x, pf.tok, pf.eid, pf.wt, plan, *lay.bank.tables(), *pf.scr, y, meta=pf.meta, npos=npos,
+                      inv=pf.inv[:2 * T], topk=2)
+        ys.append(y)
+    assert bool(ys[0].any()) and torch.equal(ys[0], ys[1])
