@@ -812,9 +812,9 @@ static int moe4t_run(const void* x, const int* tok, const float* wt, const int* 
                      const int64_t* ds, uint16_t* ar, float* d, float* out, int ps, const int* meta, int T, int xf,
                      const int* inv, int topk, uint16_t* ob, bool base, void* stream)
 {
-    if (npos == 0 && !base) return HMOE_OK;                                      // moe4t.cu:508: no pick, no work
+    if (npos == 0) return HMOE_OK;                                      // moe4t.cu:508: no pick, no work
     HMOE_REQUIRE(x && tok && wt && rbt && ar && (out || base), "moe4t_forward: null buffer");
-    HMOE_REQUIRE(npos >= 0 && nrb >= 0 && npos <= ps && T >= 1, "moe4t_forward: npos %d nrb %d ps %d T %d", npos, nrb, ps,
+    HMOE_REQUIRE(npos > 0 && nrb >= 0 && npos <= ps && T >= 1, "moe4t_forward: npos %d nrb %d ps %d T %d", npos, nrb, ps,
                  T);
     HMOE_REQUIRE((size_t) T * H * 2 <= UINT32_MAX && (size_t) ps * I * 2 <= UINT32_MAX,
                  "moe4t_forward: T %d ps %d past the 4 GB input offsets", T, ps);
@@ -908,6 +908,16 @@ extern "C" int hmoe_moe4t_forward_base_bf16(const void* x, const int* tok, const
     (void) eid; (void) gu;
     HMOE_REQUIRE(out_bf16 && inv && d && T >= 1 && ps >= 1 && ((uintptr_t) out_bf16 & 7) == 0,
                  "moe4t_forward_base_bf16: needs d, the inverse map and an 8-byte aligned bf16 output");
+    if (npos == 0)
+    {
+        // no pick: the base alone (np 0: the combine drops every pick; what it loads for them is d's first row)
+        HMOE_REQUIRE(topk >= 1 && topk <= TOPK && ((uintptr_t) base & 15) == 0 && ((uintptr_t) d & 15) == 0,
+                     "moe4t_forward_base_bf16: topk %d or alignment", topk);
+        hipStream_t st = (hipStream_t) stream;
+        if (base) pfin_kernel<PF_BASE><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, 0, -1, (float*) base, out_bf16);
+        else pfin_kernel<PF_BF16><<<T, 256, 0, st>>>((const _Float16*) d, inv, topk, 0, -1, nullptr, out_bf16);
+        return HMOE_LAUNCHED("moe4t_forward_base_bf16");
+    }
     return moe4t_run(x, tok, wt, rbt, npos, nrb, n_tab, gw, uw, dw, gs, us, ds, ar, d, (float*) base, ps, meta, T, xf, inv,
                      topk, out_bf16, true, stream);
 }

@@ -222,7 +222,7 @@ int hmoe_moe4t_forward_bf16(const void* x, const int* tok, const int* eid, const
                             uint16_t* out_bf16, void* stream);
 /* The same with a partial that is only read: out_bf16 = bf16(base + picks), base fp32 [T][H] or NULL (no partial). For the
  * layer's long prefill, the shared expert's rows from hmoe_shared_rows as the base: no fp32 buffer has to be kept
- * zeroed. d and inv are required; npos = 0 gives the base alone. */
+ * zeroed. d and inv are required; npos = 0 gives the base alone, and x, the tables and ar are not looked at. */
 int hmoe_moe4t_forward_base_bf16(const void* x, const int* tok, const int* eid, const float* wt, const int* rbt, int npos,
                                  int nrb, int n_tab, const int64_t* gw, const int64_t* uw, const int64_t* dw,
                                  const int64_t* gs, const int64_t* us, const int64_t* ds, float* gu, uint16_t* ar,

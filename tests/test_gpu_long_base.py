@@ -71,3 +71,19 @@ def test_many_row_blocks(lay, npos):
                       inv=pf.inv[:2 * T], topk=2)
         ys.append(y)
     assert bool(ys[0].any()) and torch.equal(ys[0], ys[1])
+
+
+def test_base_without_picks(lay):
+    """no pick reaches the tier: the base alone (or zeros), whatever the scratch's room, with neither tables nor act rows"""
+    from hecate_amd import _lib
+    dev = lay.device
+    T = 33
+    base = torch.randn((T, H), generator=torch.Generator().manual_seed(5)).to(dev)
+    d = torch.full((1, H), float("nan"), dtype=torch.float16, device=dev)
+    inv = torch.full((T * 8,), -1, dtype=torch.int32, device=dev)
+    out = torch.empty((T, H), dtype=torch.bfloat16, device=dev)
+    for b in (base, None):
+        out.fill_(7)
+        _lib.call("hmoe_moe4t_forward_base_bf16", *([None] * 5), 0, 0, 0, *([None] * 8), d.data_ptr(), _lib.ptr(b), 1, None, T,
+                  _lib.XF_BF16, inv.data_ptr(), 8, out.data_ptr(), _lib.stream_of(dev))
+        assert torch.equal(out, torch.zeros_like(out) if b is None else b.bfloat16())
