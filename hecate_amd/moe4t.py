@@ -44,9 +44,10 @@ def forward(x, tok, eid, wt, rbt, gw, uw, dw, gs, us, ds, gu, ar, d, out, meta=N
     nrb = rbt.shape[0] if nrb is None else int(nrb)
     ps = ar.shape[0]
     # d: the reference's fp32 [1, ps, H] (moe4t.scratch) or an f16 [ps, H] buffer: the kernels write f16 rows into it
-    # (the copy of bf16 x, then with inv each pick's down row), ps * H * 2 bytes
+    # (the copy of bf16 x, then with inv each pick's down row): ps rows, or T if x is bf16 and its copy is the longer
+    drows = max(ps, T) if x.dtype == torch.bfloat16 else ps
     if npos > ps or ar.shape[1] != I or ar.dtype != torch.float16 or d.dtype not in (torch.float32, torch.float16) \
-            or d.numel() * d.element_size() < ps * H * 2 or not d.is_contiguous():
+            or d.numel() * d.element_size() < drows * H * 2 or not d.is_contiguous():
         raise RuntimeError(f"moe4t: scratch for {ps} picks, {npos} given")
     if out_bf16 is not None:
         if inv is None or out_bf16.dtype != torch.bfloat16 or not out_bf16.is_contiguous() \
