@@ -4,9 +4,10 @@
 // Dispatch: picks sorted by (expert, flat index) by a counting sort with per-block histograms and in-block ranks, so
 // the order equals a stable argsort of the selection; row blocks {expert, first pick, picks, 0} of at most bm picks.
 // GEMMs: workgroup = (row block of picks of one expert, 128 gate/up or 256 down output columns); see pgemm.h, and
-// pgemm16_kernel for the long prefill. gu fuses act = silu(g) * u * w (f16), down writes d = W_d act (fp32), fin adds each
-// token's picks into out in top-k order (or with atomics, as p4_fin_kernel, when no inverse map is given). The shared
-// expert's projections ride in the same launches (moe4p) or run on the dense MFMA GEMMs of shared_gemm.hip.
+// pgemm16_kernel for long chunks of many picks an expert. gu fuses act = silu(g) * u * w (f16), down writes d = W_d act as
+// f16 rows, whose picks fin sums per token in top-k order in fp32 (or, when no inverse map is given, down adds its fp32 sums
+// into out with atomics, as p4_fin_kernel). The shared expert's projections ride in the same launches (moe4p up to 4096
+// tokens) or run on the dense MFMA GEMMs of shared_gemm.hip.
 #include "pgemm.h"
 
 namespace hmoe {
@@ -230,10 +231,10 @@ __global__ void __launch_bounds__(DS_W * 64) disp_one_kernel(
 // ---------------------------------------------------------------------------------------------------------------
 // grouped GEMMs
 // ---------------------------------------------------------------------------------------------------------------
-// The long prefill's grouped GEMM for both projections (blocks of up to 256 picks in one pass; the other chunks run on
-// pgemm.h's). Workgroup = (row block of <= 256 picks of one expert, 64 NS output columns), 8 waves; wave w of column block
-// cb owns output strips nb0 = NWV NS cb + NS w .. + NS (16 rows each) of NMAT matrices (gate and up: NS = 1, down: NS = 2),
-// so every dequantised fragment feeds up to 16 pick tiles. Per 128-k group kg:
+// The grouped GEMM of chunks of many picks an expert, for both projections (the rule is in moe4t_run; every other chunk runs
+// on pgemm.h's): blocks of up to 256 picks in one pass. Workgroup = (row block of one expert, 128 NS output columns), 8
+// waves; wave w of column block cb owns output strips nb0 = NWV NS cb + NS w .. + NS (16 rows each) of NMAT matrices (gate
+// and up: NS = 1, down: NS = 2), so every dequantised fragment feeds up to 16 pick tiles. Per 128-k group kg:
 //   * the block's input rows are staged in LDS as f16 by direct global-to-LDS loads (double-buffered, one barrier
 //     per group): the next group's rows load while this group computes;
 //   * the weight tiles come from a ring of D groups of unconditional 16-byte loads, issued D - 1 groups ahead, so HBM
@@ -249,263 +250,242 @@ struct PFetch
     u32x4 q[NS][NMAT];
 };
 
-// NTT: 16-pick tiles per pass; NWV waves, each staging two tiles
-template <int NMAT, int NS, int D, int EPI, int NTT = 16, int NWV = 8>
-__global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(2))) pgemm16_kernel(
+template <int NMAT, int EPI>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) pgemm16_kernel(
     const _Float16* __restrict__ xin, const int* __restrict__ tok, const float* __restrict__ wt,
     const int* __restrict__ rbt, int nrb, const int* __restrict__ meta, int n_tab,
     const int64_t* __restrict__ w0, const int64_t* __restrict__ w1, const int64_t* __restrict__ s0,
-    const int64_t* __restrict__ s1, _Float16* __restrict__ ar, float* __restrict__ dout, int T, int off, int np,
-    float* __restrict__ fout = nullptr, int ps = 0)
+    const int64_t* __restrict__ s1, void* __restrict__ out, int T, int np)
 {
-    static_assert((NMAT == 2) == (EPI == EPI_ACT || EPI == EPI_RAW), "gate/up epilogues need both matrices");
+    static_assert((NMAT == 2) == (EPI == EPI_ACT), "gate/up's epilogue needs both matrices");
     constexpr int K = NMAT == 2 ? H : I;                 // gate/up: x [T][H] -> act; down: act [.][I] -> d
     constexpr int NOUT = NMAT == 2 ? I : H;
     constexpr int KG = K / 128;
+    constexpr int NTT = 16, NWV = 8, NS = 2 / NMAT, D = 4;      // pick tiles, waves (two tiles staged by each), ring depth
     static_assert(KG % D == 0, "the ring depth divides the k groups");
-    static_assert(NS * NMAT * NTT == 32, "32 accumulator tiles per wave (4 fragments x 8 tiles or 2 x 16)");
-    static_assert(NTT == 2 * NWV, "each wave stages two tiles");
-    constexpr int PBX = 16 * NTT;                        // picks per pass
+    static_assert(16 * NTT == 2 * PB, "a block is one pass (get_block's limit)");
     // the staged input of a 128-k group (four 1 KB blocks per 16-pick tile, below); two buffers, the next group loads
     // while one computes
     __shared__ __attribute__((aligned(16))) u32x4 xs0[NTT * 4 * 64];
     __shared__ __attribute__((aligned(16))) u32x4 xs1[NTT * 4 * 64];
     int rbi, cbi;
     xcd_tile(pgemm_index((nrb + 7) & ~7), rbi, cbi, NOUT / (16 * NS * NWV));
-    Block rb;
-    if (!get_block(rbt, nrb, meta, n_tab, np, rbi, rb)) return;
-    // a block of more than PBX picks runs as passes of PBX, one after the other (a later pass reads the weights
-    // again, mostly from the caches); the barrier between them keeps one pass's last LDS reads ahead of the next
-    // pass's first staging
-    for (int h0 = 0; h0 < rb.rows; h0 += PBX)
+    Block b;
+    if (!get_block(rbt, nrb, meta, n_tab, np, rbi, b)) return;
+    const int t = threadIdx.x, l = t & 63, row = l & 15;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);   // wave index, kept in a scalar register
+    const int nb0 = (cbi * NWV + w) * NS;
+    const uint8_t* wp[NMAT];
+    const uint8_t* sp[NMAT];
+    #pragma unroll
+    for (int m = 0; m < NMAT; ++m)
     {
-        if (h0) __syncthreads();
-        const Block b = {rb.e, rb.p0 + h0, min(PBX, rb.rows - h0)};
-        const int t = threadIdx.x, l = t & 63, row = l & 15;
-        const int w = __builtin_amdgcn_readfirstlane(t >> 6);   // wave index, kept in a scalar register
-        const int nb0 = (cbi * NWV + w) * NS;
-        const uint8_t* wp[NMAT];
-        const uint8_t* sp[NMAT];
+        wp[m] = (const uint8_t*) (m == 0 ? w0 : w1)[b.e];
+        sp[m] = (const uint8_t*) (m == 0 ? s0 : s1)[b.e];
+    }
+    const int ntt = (b.rows + 15) >> 4;
+    // (without it the first tile of every k step is tested too: 4600 to 8192 tokens 2.5 % slower)
+    __builtin_assume(ntt >= 1);                             // (get_block's promise, which it does not carry here)
+    const DqConsts dq = dq_consts();
+    // The staged input of a 128-k group: per 16-pick tile, four 1 KB blocks (k half kh, row half rh) of 8 rows x 64
+    // k; lane l of a block takes row l / 8's 16-byte chunk (l % 8) ^ (l / 8) (whole 128-byte lines from memory) and
+    // stores it at 16 l, so a fragment read (row l % 16, chunk 4 (k % 2) + l / 16 of k half k / 2) meets distinct
+    // banks. Wave w stages tiles 2w and 2w + 1: lane l's source row in each row half; a pick past the block re-reads
+    // a valid row (its output columns are never stored), a whole tile past the block reads one fixed 16 bytes.
+    uint32_t src[2][2];                                     // byte offsets from xin
+    #pragma unroll
+    for (int h = 0; h < 2; ++h)
         #pragma unroll
-        for (int m = 0; m < NMAT; ++m)
+        for (int rh = 0; rh < 2; ++rh)
         {
-            wp[m] = (const uint8_t*) (m == 0 ? w0 : w1)[b.e];
-            sp[m] = (const uint8_t*) (m == 0 ? s0 : s1)[b.e];
+            const int tt = 2 * w + h, pk = tt * 16 + 8 * rh + (l >> 3);
+            const bool in = pk < b.rows, tin = tt < ntt;
+            int srow = b.p0 + (in ? pk : 0);
+            if (NMAT == 2)
+            {
+                const int tk = tok[srow];
+                srow = (unsigned) tk < (unsigned) T ? tk : 0;
+            }
+            src[h][rh] = (uint32_t) (((size_t) srow * K + (tin ? 8 * ((l & 7) ^ (l >> 3)) : 0)) * 2);
         }
-        const int ntt = (b.rows + 15) >> 4;
-        const DqConsts dq = dq_consts();
-        // The staged input of a 128-k group: per 16-pick tile, four 1 KB blocks (k half kh, row half rh) of 8 rows x 64
-        // k; lane l of a block takes row l / 8's 16-byte chunk (l % 8) ^ (l / 8) (whole 128-byte lines from memory) and
-        // stores it at 16 l, so a fragment read (row l % 16, chunk 4 (k % 2) + l / 16 of k half k / 2) meets distinct
-        // banks. Wave w stages tiles 2w and 2w + 1: lane l's source row in each row half; a pick past the block re-reads
-        // a valid row (its output columns are never stored), a whole tile past the block reads one fixed 16 bytes.
-        uint32_t src[2][2];                                     // byte offsets from xin
+    int fo[4];
+    #pragma unroll
+    for (int k = 0; k < 4; ++k)
+        fo[k] = ((k >> 1) * 2 + (row >> 3)) * 64 + 8 * (l & 7) + ((4 * (k & 1) + (l >> 4)) ^ (l & 7));
+    // Direct global-to-LDS loads (16 bytes per lane, lane l at LDS base + 16 l), issued from inline assembly: the
+    // compiler then does not count them, so its own waits for the weight ring stay exact, and the wait that makes a
+    // staged group visible is placed by hand before the barrier (the loads issued after a stage are exactly those
+    // of one ring refill). M0 holds the LDS base of each load; nothing else in this kernel uses M0.
+    auto stage = [&](int kg, u32x4* buf) {
         #pragma unroll
         for (int h = 0; h < 2; ++h)
+        {
+            const int tt = 2 * w + h;
+            const bool tin = tt < ntt;
             #pragma unroll
-            for (int rh = 0; rh < 2; ++rh)
-            {
-                const int tt = 2 * w + h, pk = tt * 16 + 8 * rh + (l >> 3);
-                const bool in = pk < b.rows, tin = tt < ntt;
-                int srow;
-                if (NMAT == 2)
-                {
-                    // (no token map: the picks' inputs are rows p0 .. of xin, as the moe4t test entry passes them)
-                    const int tk = !tok ? b.p0 + (in ? pk : 0) : tok[b.p0 + (in ? pk : 0)];
-                    srow = (unsigned) tk < (unsigned) T ? tk : 0;
-                }
-                else srow = off + b.p0 + (in ? pk : 0);
-                src[h][rh] = (uint32_t) (((size_t) srow * K + (tin ? 8 * ((l & 7) ^ (l >> 3)) : 0)) * 2);
-            }
-        int fo[4];
-        #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            fo[k] = ((k >> 1) * 2 + (row >> 3)) * 64 + 8 * (l & 7) + ((4 * (k & 1) + (l >> 4)) ^ (l & 7));
-        // Direct global-to-LDS loads (16 bytes per lane, lane l at LDS base + 16 l), issued from inline assembly: the
-        // compiler then does not count them, so its own waits for the weight ring stay exact, and the wait that makes a
-        // staged group visible is placed by hand before the barrier (the loads issued after a stage are exactly those
-        // of one ring refill). M0 holds the LDS base of each load; nothing else in this kernel uses M0.
-        auto stage = [&](int kg, u32x4* buf) {
-            #pragma unroll
-            for (int h = 0; h < 2; ++h)
-            {
-                const int tt = 2 * w + h;
-                const bool tin = tt < ntt;
+            for (int kh = 0; kh < 2; ++kh)
                 #pragma unroll
-                for (int kh = 0; kh < 2; ++kh)
-                    #pragma unroll
-                    for (int rh = 0; rh < 2; ++rh)
-                    {
-                        const uint32_t gp = src[h][rh] + (tin ? (kg * 128 + 64 * kh) * 2 : 0);
-                        const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t)
-                            (__attribute__((address_space(3))) void*) (buf + (tt * 4 + kh * 2 + rh) * 64));
-    #pragma clang diagnostic push
-    #pragma clang diagnostic ignored "-Winline-asm"
-                        // (an SALU write of M0 needs one wait state before an LDS-DMA load reads it: the s_nop)
-                        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(gp), "s"(xin),
-                                     "s"(lds) : "memory", "m0");
-    #pragma clang diagnostic pop
-                    }
+                for (int rh = 0; rh < 2; ++rh)
+                {
+                    const uint32_t gp = src[h][rh] + (tin ? (kg * 128 + 64 * kh) * 2 : 0);
+                    const uint32_t lds = __builtin_amdgcn_readfirstlane((uint32_t) (uintptr_t)
+                        (__attribute__((address_space(3))) void*) (buf + (tt * 4 + kh * 2 + rh) * 64));
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+                    // (an SALU write of M0 needs one wait state before an LDS-DMA load reads it: the s_nop)
+                    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(gp), "s"(xin),
+                                 "s"(lds) : "memory", "m0");
+#pragma clang diagnostic pop
+                }
+        }
+    };
+    PFetch<NMAT, NS> ring[D];
+    // the row scales of two blocks of 4 groups (a block's 4 bf16 of one row are 8 contiguous bytes of I4G128)
+    u32x2 sc4[2][NS][NMAT];
+    // the weights of group kg into ring slot SL; when kg starts a block of 4, the block's scales too, into sc4[SC]
+    // (SC = -1: none). Offsets are 32-bit (an expert's matrix is 6.3 MB), so the loads take the base from scalar
+    // registers.
+    auto fetch = [&](int kg, auto sl, auto sc) {
+        constexpr int SL = decltype(sl)::value, SC = decltype(sc)::value;
+        #pragma unroll
+        for (int st = 0; st < NS; ++st)
+            #pragma unroll
+            for (int m = 0; m < NMAT; ++m)
+            {
+                const int nb = nb0 + st;
+                ring[SL].q[st][m] = ldw16(wp[m] + (uint32_t) (((nb * KG + kg) * 64 + l) * 16));
+                if constexpr (SC >= 0)
+                    sc4[SC][st][m] = ld8(sp[m] + (uint32_t) (sc_index(nb * 16 + row, kg & ~3, KG) * 2));
             }
-        };
-        PFetch<NMAT, NS> ring[D];
-        // the row scales of two blocks of 4 groups (a block's 4 bf16 of one row are 8 contiguous bytes of I4G128)
-        u32x2 sc4[2][NS][NMAT];
-        // the weights of group kg into ring slot SL; when kg starts a block of 4, the block's scales too, into sc4[SC]
-        // (SC = -1: none). Offsets are 32-bit (an expert's matrix is 6.3 MB), so the loads take the base from scalar
-        // registers.
-        auto fetch = [&](int kg, auto sl, auto sc) {
-            constexpr int SL = decltype(sl)::value, SC = decltype(sc)::value;
+    };
+    f32x4 acc[NS][NMAT][NTT];
+    #pragma unroll
+    for (int st = 0; st < NS; ++st)
+        #pragma unroll
+        for (int m = 0; m < NMAT; ++m)
+            #pragma unroll
+            for (int tt = 0; tt < NTT; ++tt) acc[st][m][tt] = (f32x4) {0.f, 0.f, 0.f, 0.f};
+    // the prologue stages group 0 and fills D - 1 ring slots; group kg then issues its loads (the next stage and
+    // the refill of the slot group kg - 1 used, D - 1 groups ahead) only after its own operands are in hand, so
+    // that no wait for them counts the new loads: a weight refill has D - 1 groups to arrive
+    stage(0, xs0);
+    static_for<D - 1>([&](auto sc) {
+        constexpr int g = decltype(sc)::value;
+        fetch(g, sc, std::integral_constant<int, g % 4 == 0 ? (g / 4) % 2 : -1>{});
+        __builtin_amdgcn_sched_barrier(0);                  // keep the ring's issue order (waits count in order)
+    });
+    // the group loop runs in steps of 8, so that the ring slot (kg % D), the scale block (kg / 4 % 2) and whether a
+    // refill starts a block are compile-time constants
+    static_assert(KG % 8 == 0 && 8 % D == 0, "the group loop runs in steps of 8");
+    for (int kg0 = 0; kg0 < KG; kg0 += 8)
+    {
+        static_for<8>([&](auto sc8) {
+            constexpr int s8 = decltype(sc8)::value, s = s8 % D;
+            const int kg = kg0 + s8;
+            const bool even = (kg & 1) == 0;
+            u32x4* cur = even ? xs0 : xs1;
+            // this wave's staged loads of group kg are older than the loads of the refill issued with them in group
+            // kg - 1 (its NS NMAT weight loads and, when that refill started a block of 4, as many scale loads); for
+            // kg = 0 every load is waited for. The barrier then makes every wave's group kg visible.
+            constexpr int gp = (s8 + 7) % 8 + D - 1;            // the group refilled in group kg - 1, mod 8
+            constexpr int after = NS * NMAT * (gp % 4 == 0 ? 2 : 1);
+            if (kg == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(after) : "memory");
+            __syncthreads();
+            // the slot's scales and first k step: the compiler's wait for the slot falls here, before the loads
+            // below (its count of later loads is then the D - 2 refills it knows of, and the stage, which has
+            // arrived, is the only load it does not count)
+            f16x2 sh[NS][NMAT];
+            f16x8 a0[NS][NMAT];
             #pragma unroll
             for (int st = 0; st < NS; ++st)
                 #pragma unroll
                 for (int m = 0; m < NMAT; ++m)
                 {
-                    const int nb = nb0 + st;
-                    ring[SL].q[st][m] = ldw16(wp[m] + (uint32_t) (((nb * KG + kg) * 64 + l) * 16));
-                    if constexpr (SC >= 0)
-                        sc4[SC][st][m] = ld8(sp[m] + (uint32_t) (sc_index(nb * 16 + row, kg & ~3, KG) * 2));
+                    const uint32_t sw = sc4[s8 / 4][st][m][(s8 % 4) / 2];     // bf16 of group kg: half s8 % 2
+                    const _Float16 h = (_Float16) __uint_as_float(s8 % 2 == 0 ? sw << 16 : sw & 0xffff0000u);
+                    sh[st][m] = (f16x2) {h, h};
+                    a0[st][m] = dq8s(ring[s].q[st][m][0], sh[st][m], dq);
                 }
-        };
-        f32x4 acc[NS][NMAT][NTT];
-        #pragma unroll
-        for (int st = 0; st < NS; ++st)
+            __builtin_amdgcn_sched_barrier(0);
+            if (kg + 1 < KG) stage(kg + 1, even ? xs1 : xs0);
+            // the refill: group kg + D - 1, clamped to the last group; it starts a block of 4 when (s8 + D - 1) % 4
+            // == 0, whose scales go to sc4[(s8 + D - 1) / 4 % 2] (kg0 is a multiple of 8). Past the last group the
+            // clamped group's block is loaded again into the buffer that no remaining group reads.
+            constexpr int gn = s8 + D - 1;
+            fetch(min(kg + D - 1, KG - 1), std::integral_constant<int, (s + D - 1) % D>{},
+                  std::integral_constant<int, gn % 4 == 0 ? (gn / 4) % 2 : -1>{});
+            __builtin_amdgcn_sched_barrier(0);
             #pragma unroll
-            for (int m = 0; m < NMAT; ++m)
-                #pragma unroll
-                for (int tt = 0; tt < NTT; ++tt) acc[st][m][tt] = (f32x4) {0.f, 0.f, 0.f, 0.f};
-        // the prologue stages group 0 and fills D - 1 ring slots; group kg then issues its loads (the next stage and
-        // the refill of the slot group kg - 1 used, D - 1 groups ahead) only after its own operands are in hand, so
-        // that no wait for them counts the new loads: a weight refill has D - 1 groups to arrive
-        stage(0, xs0);
-        static_for<D - 1>([&](auto sc) {
-            constexpr int g = decltype(sc)::value;
-            fetch(g, sc, std::integral_constant<int, g % 4 == 0 ? (g / 4) % 2 : -1>{});
-            __builtin_amdgcn_sched_barrier(0);                  // keep the ring's issue order (waits count in order)
-        });
-        // the group loop runs in steps of 8, so that the ring slot (kg % D), the scale block (kg / 4 % 2) and whether a
-        // refill starts a block are compile-time constants
-        static_assert(KG % 8 == 0 && 8 % D == 0, "the group loop runs in steps of 8");
-        for (int kg0 = 0; kg0 < KG; kg0 += 8)
-        {
-            static_for<8>([&](auto sc8) {
-                constexpr int s8 = decltype(sc8)::value, s = s8 % D;
-                const int kg = kg0 + s8;
-                const bool even = (kg & 1) == 0;
-                u32x4* cur = even ? xs0 : xs1;
-                // this wave's staged loads of group kg are older than the loads of the refill issued with them in group
-                // kg - 1 (its NS NMAT weight loads and, when that refill started a block of 4, as many scale loads); for
-                // kg = 0 every load is waited for. The barrier then makes every wave's group kg visible.
-                constexpr int gp = (s8 + 7) % 8 + D - 1;            // the group refilled in group kg - 1, mod 8
-                constexpr int after = NS * NMAT * (gp % 4 == 0 ? 2 : 1);
-                if (kg == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(after) : "memory");
-                __syncthreads();
-                // the slot's scales and first k step: the compiler's wait for the slot falls here, before the loads
-                // below (its count of later loads is then the D - 2 refills it knows of, and the stage, which has
-                // arrived, is the only load it does not count)
-                f16x2 sh[NS][NMAT];
-                f16x8 a0[NS][NMAT];
+            for (int k = 0; k < 4; ++k)
+            {
+                f16x8 a[NS][NMAT];
                 #pragma unroll
                 for (int st = 0; st < NS; ++st)
                     #pragma unroll
                     for (int m = 0; m < NMAT; ++m)
-                    {
-                        const uint32_t sw = sc4[s8 / 4][st][m][(s8 % 4) / 2];     // bf16 of group kg: half s8 % 2
-                        const _Float16 h = (_Float16) __uint_as_float(s8 % 2 == 0 ? sw << 16 : sw & 0xffff0000u);
-                        sh[st][m] = (f16x2) {h, h};
-                        a0[st][m] = dq8s(ring[s].q[st][m][0], sh[st][m], dq);
-                    }
-                __builtin_amdgcn_sched_barrier(0);
-                if (kg + 1 < KG) stage(kg + 1, even ? xs1 : xs0);
-                // the refill: group kg + D - 1, clamped to the last group; it starts a block of 4 when (s8 + D - 1) % 4
-                // == 0, whose scales go to sc4[(s8 + D - 1) / 4 % 2] (kg0 is a multiple of 8). Past the last group the
-                // clamped group's block is loaded again into the buffer that no remaining group reads.
-                constexpr int gn = s8 + D - 1;
-                fetch(min(kg + D - 1, KG - 1), std::integral_constant<int, (s + D - 1) % D>{},
-                      std::integral_constant<int, gn % 4 == 0 ? (gn / 4) % 2 : -1>{});
-                __builtin_amdgcn_sched_barrier(0);
+                        a[st][m] = k == 0 ? a0[st][m] : dq8s(ring[s].q[st][m][k], sh[st][m], dq);
+                // The pick tiles are read two tiles ahead of their MFMAs (a tile past the block reads stale LDS data, never
+                // used). Each read is consumed by an empty asm after the MFMAs of the tile before it, which keeps the
+                // read ahead of the branch that ends the block's tiles: the compiler would otherwise sink it behind that
+                // branch, next to its MFMAs, and wait out its latency there (-8 % at 8192 tokens; pinning the asm behind
+                // the MFMAs cost 1.5 %).
+                constexpr int PD = 2;
+                f16x8 bq[PD + 1];
                 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+                for (int i = 0; i < PD; ++i) bq[i] = as_f16x8(cur[i * 256 + fo[k]]);
+                #pragma unroll
+                for (int tt = 0; tt < NTT; ++tt)
                 {
-                    f16x8 a[NS][NMAT];
+                    if (tt >= ntt) break;
+                    if (tt + PD < NTT) bq[PD] = as_f16x8(cur[(tt + PD) * 256 + fo[k]]);
                     #pragma unroll
                     for (int st = 0; st < NS; ++st)
                         #pragma unroll
-                        for (int m = 0; m < NMAT; ++m)
-                            a[st][m] = k == 0 ? a0[st][m] : dq8s(ring[s].q[st][m][k], sh[st][m], dq);
-                    // The pick tiles are read PD tiles ahead of their MFMAs (a tile past the block reads stale LDS
-                    // data, never used). Each read is consumed by an empty asm after the MFMAs of the tile before it,
-                    // which keeps the read ahead of the branch that ends the block's tiles: the compiler would
-                    // otherwise sink it behind that branch, next to its MFMAs, and wait out its latency there. With
-                    // four MFMAs per tile one tile ahead is enough and the consuming asm is pinned behind all four
-                    // (measured: -1 %); with two, two tiles ahead and the asm left to the scheduler (-8 % at 8192
-                    // tokens, pinning it cost 1.5 %).
-                    constexpr int PD = NS * NMAT >= 4 ? 1 : 2;
-                    f16x8 bq[PD + 1];
+                        for (int m = 0; m < NMAT; ++m) acc[st][m][tt] = mfma16(a[st][m], bq[0], acc[st][m][tt]);
+                    if (tt + 1 < NTT) asm volatile("" :: "v"(bq[1]));
                     #pragma unroll
-                    for (int i = 0; i < PD; ++i) bq[i] = as_f16x8(cur[i * 256 + fo[k]]);
-                    #pragma unroll
-                    for (int tt = 0; tt < NTT; ++tt)
-                    {
-                        if (tt >= ntt) break;
-                        if (tt + PD < NTT) bq[PD] = as_f16x8(cur[(tt + PD) * 256 + fo[k]]);
-                        #pragma unroll
-                        for (int st = 0; st < NS; ++st)
-                            #pragma unroll
-                            for (int m = 0; m < NMAT; ++m) acc[st][m][tt] = mfma16(a[st][m], bq[0], acc[st][m][tt]);
-                        if constexpr (PD == 1) __builtin_amdgcn_sched_barrier(0);
-                        if (tt + 1 < NTT) asm volatile("" :: "v"(bq[1]));
-                        #pragma unroll
-                        for (int i = 0; i < PD; ++i) bq[i] = bq[i + 1];
-                    }
+                    for (int i = 0; i < PD; ++i) bq[i] = bq[i + 1];
                 }
-            });
-        }
-        // epilogue: lane holds output rows 4(l/16)..+4 of pick tt*16 + l%16
+            }
+        });
+    }
+    // epilogue: lane holds output rows 4(l/16)..+4 of pick tt*16 + l%16
+    #pragma unroll
+    for (int tt = 0; tt < NTT; ++tt)
+    {
+        const int pk = tt * 16 + row;
+        if (pk >= b.rows) continue;
         #pragma unroll
-        for (int tt = 0; tt < NTT; ++tt)
+        for (int st = 0; st < NS; ++st)
         {
-            const int pk = tt * 16 + row;
-            if (pk >= b.rows) continue;
-            #pragma unroll
-            for (int st = 0; st < NS; ++st)
+            const int n = (nb0 + st) * 16 + 4 * (l >> 4);
+            if (EPI == EPI_ACT)
             {
-                const int n = (nb0 + st) * 16 + 4 * (l >> 4);
-                if (EPI == EPI_RAW)
+                const float wv = wt[b.p0 + pk];
+                _Float16 o[4];
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (_Float16) (silu(acc[st][0][tt][i]) * acc[st][NMAT - 1][tt][i] * wv);
+                *(uint2*) ((_Float16*) out + (size_t) (b.p0 + pk) * NOUT + n) = *(const uint2*) o;
+            }
+            else if (EPI == EPI_FIN)
+            {
+                // out[tok] += acc (the combine in the epilogue, fp32 atomics as moe4t.cu's down GEMM: no d buffer)
+                const int tk = tok[b.p0 + pk];
+                if ((unsigned) tk < (unsigned) T)
                 {
+                    float* o = (float*) out + (size_t) tk * NOUT + n;
                     #pragma unroll
-                    for (int m = 0; m < NMAT; ++m)
-                        *(f32x4*) (dout + ((size_t) m * ps + b.p0 + pk) * NOUT + n) = acc[st][m][tt];
+                    for (int i = 0; i < 4; ++i) unsafeAtomicAdd(o + i, acc[st][0][tt][i]);
                 }
-                else if (EPI == EPI_ACT)
-                {
-                    const float wv = wt[b.p0 + pk];
-                    _Float16 o[4];
-                    #pragma unroll
-                    for (int i = 0; i < 4; ++i) o[i] = (_Float16) (silu(acc[st][0][tt][i]) * acc[st][NMAT - 1][tt][i] * wv);
-                    *(uint2*) (ar + (size_t) (off + b.p0 + pk) * NOUT + n) = *(const uint2*) o;
-                }
-                else if (EPI == EPI_FIN)
-                {
-                    // out[tok] += acc (the combine in the epilogue, fp32 atomics as moe4t.cu's down GEMM: no d buffer)
-                    const int tk = tok[b.p0 + pk];
-                    if ((unsigned) tk < (unsigned) T)
-                    {
-                        float* o = fout + (size_t) tk * NOUT + n;
-                        #pragma unroll
-                        for (int i = 0; i < 4; ++i) unsafeAtomicAdd(o + i, acc[st][0][tt][i]);
-                    }
-                }
-                else if (EPI == EPI_D16)
-                {
-                    // (a pick's down row rounded to f16: half the bytes written here and read by the combine)
-                    _Float16 o[4];
-                    #pragma unroll
-                    for (int i = 0; i < 4; ++i) o[i] = (_Float16) acc[st][0][tt][i];
-                    *(uint2*) ((_Float16*) dout + (size_t) (off + b.p0 + pk) * NOUT + n) = *(const uint2*) o;
-                }
-                else *(f32x4*) (dout + (size_t) (off + b.p0 + pk) * NOUT + n) = acc[st][0][tt];
+            }
+            else
+            {
+                // (a pick's down row rounded to f16: half the bytes written here and read by the combine)
+                _Float16 o[4];
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (_Float16) acc[st][0][tt][i];
+                *(uint2*) ((_Float16*) out + (size_t) (b.p0 + pk) * NOUT + n) = *(const uint2*) o;
             }
         }
     }
@@ -834,11 +814,13 @@ static int moe4t_run(const void* x, const int* tok, const float* wt, const int* 
         xh = (const _Float16*) d;
     }
     // Which grouped GEMM, by the picks an expert has on average (npos counts those outside the window too, so for a partial
-    // window the line comes earlier). pgemm16_kernel runs a whole 256-pick block in one pass, but always stages, reads and
-    // loops for 16 tiles; pgemm.h's pass follows the block's tiles and takes a longer block as two. Gate/up + down, 256
-    // experts, us: 2100 tokens 1248 + 692 against 959 + 525, 3000: 1444 + 816 against 1193 + 667, 4096 (128 picks an expert):
-    // 1713 + 954 against 1659 + 923, 6000 (188): 2188 + 1249 against 2244 + 1250, 8192 (256): 3105 + 1726 against 3236 + 1792;
-    // whole layer 4300 tokens (134) 3615 against 3582, 4600 (144) 3766 against 3816.
+    // window the line comes earlier). pgemm16_kernel runs a whole 256-pick block in one pass, but always stages for 16
+    // tiles; pgemm.h's pass follows the block's tiles and takes a longer block as two. Whole calls, 256 experts, us, pgemm16
+    // against pgemm.h: even popularity 2100 tokens 1986, 1549; 3000 2331, 1870; 4000 (125 picks an expert) 2868, 2656; 4224
+    // (132) 2978, 2908; 4300 (134) 3006, 2979; 4400 (138) 3067, 3101; 4600 3134, 3237; 6000 3789, 3805; 8192 5397, 5608.
+    // Uneven chunks (popularity as rank^-1.1 under the router's own spread) gain on pgemm.h throughout, their many small
+    // blocks outweighing the ones cut in two: 3000 tokens 2691, 2448; 4224 3620, 3428; 8192 5736, 5503. Only where all tokens
+    // pick the same few experts is it behind below the line (8 experts, 2100 tokens: 1208, 1298); that the host cannot see.
     if (nrb > 0 && npos <= 132 * n_tab)
     {
         PgArgs g{};
@@ -854,15 +836,15 @@ static int moe4t_run(const void* x, const int* tok, const float* wt, const int* 
     {
         // 256-pick blocks in one pass: 8 waves, each one 16-row strip of gate and of up (or two of down) against the
         // block's 16 pick tiles
-        pgemm16_kernel<2, 1, 4, EPI_ACT><<<pgemm_grid(nrb, I / 128), 512, 0, st>>>(xh, tok, wt, rbt, nrb, meta, n_tab,
-            gw, uw, gs, us, (_Float16*) ar, nullptr, T, 0, npos);
+        pgemm16_kernel<2, EPI_ACT><<<pgemm_grid(nrb, I / 128), 512, 0, st>>>(xh, tok, wt, rbt, nrb, meta, n_tab, gw, uw, gs, us,
+            ar, T, npos);
         // (d held the f16 copy of x, which the gate/up GEMM has consumed by now: the down rows may overwrite it)
         if (inv)
-            pgemm16_kernel<1, 2, 4, EPI_D16><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar,
-                nullptr, nullptr, rbt, nrb, meta, n_tab, dw, nullptr, ds, nullptr, nullptr, d, T, 0, npos);
+            pgemm16_kernel<1, EPI_D16><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar, nullptr, nullptr, rbt,
+                nrb, meta, n_tab, dw, nullptr, ds, nullptr, d, T, npos);
         else
-            pgemm16_kernel<1, 2, 4, EPI_FIN><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar, tok,
-                nullptr, rbt, nrb, meta, n_tab, dw, nullptr, ds, nullptr, nullptr, nullptr, T, 0, npos, out);
+            pgemm16_kernel<1, EPI_FIN><<<pgemm_grid(nrb, H / 256), 512, 0, st>>>((const _Float16*) ar, tok, nullptr, rbt, nrb,
+                meta, n_tab, dw, nullptr, ds, nullptr, out, T, npos);
     }
     // The base form neither zeroes the partial here nor reads it in the shared expert's down GEMM; both are HBM-bound on
     // these rows (8192 tokens: 244 -> 220 us here, 280 -> 244 us there, rocprofv3 averages)
