@@ -1,6 +1,6 @@
-"""The grouped expert GEMM at every pick-tile count and its edges: one expert with n picks (and a neighbour with 3), through
-the device dispatch and moe4p.forward, against a torch fp32 reference on the same dequantised weights; and the shared
-expert in the same launches at the edges of its token blocks."""
+"""The grouped expert GEMMs at every pick-tile count and their edges: one expert with n picks (and a neighbour with 3), through
+the device dispatch and moe4p.forward or, on either side of its rule, moe4t.forward, against a torch fp32 reference on the
+same dequantised weights; and the shared expert in the same launches at the edges of its token blocks."""
 import pytest
 import torch
 
@@ -108,3 +108,52 @@ def test_shared_apart(lay):
                       npos=T, nrb=pf.nrb_max, shared=lay.shared_rows())
         ys.append(y)
     assert bool(ys[1].abs().amax(1).all()) and torch.equal(ys[0].view(torch.int32), ys[1][:4096].view(torch.int32))
+
+
+@pytest.mark.parametrize("ordered", (True, False))
+@pytest.mark.parametrize("room", (264, 265))
+@pytest.mark.parametrize("n", NS[:-2] + (239, 240, 241, 255, 256))
+def test_moe4t_pick_counts(lay, n, room, ordered):
+    """moe4t.forward on both of its kernels: 132 picks an expert is the last bound on the picks (264 for 2 experts) that
+    takes the tile-count GEMM, and one more takes the one of 16 tiles a pass, which cuts no block of up to 256"""
+    from hecate_amd import moe4t, synth, tier
+    from torchref import moe_rows
+    dev = lay.device
+    T = n + 3
+    x = synth.gen_x(500 + n, T, dev)
+    sel = torch.zeros((T, 1), dtype=torch.int64, device=dev)
+    sel[torch.arange(3, device=dev) * (T // 3)] = 1
+    rw = (0.25 + 0.5 * torch.rand((T, 1), generator=torch.Generator().manual_seed(n))).half().to(dev)
+    pf = tier.PrefillBuffers(room, 1, 0, 2, 256, dev, bm=256, long=True).run(sel, rw)
+    y = torch.zeros((T, 6144), dtype=torch.float32, device=dev)
+    moe4t.forward(x, pf.tok, pf.eid, pf.wt, pf.rbt, *lay.bank.tables(), *pf.scr, y, meta=pf.meta, npos=room, nrb=pf.nrb_max,
+                  inv=pf.inv[:T] if ordered else None, topk=1)
+    assert int(pf.meta[1].item()) == 2
+    ref = moe_rows(lay, x, sel, rw, with_shared=False)
+    worst = ((y - ref).abs() / bound(ref)).max().item()
+    assert worst <= 1.0, (n, room, ordered, worst)
+
+
+@pytest.mark.parametrize("ordered", (True, False))
+def test_moe4t_skewed_blocks(lay, ordered):
+    """the 16-tile GEMM on an uneven plan: one expert cut into blocks of 205, one of 40 picks, tokens with both, one or none"""
+    from hecate_amd import moe4t, synth, tier
+    from torchref import moe_rows
+    dev = lay.device
+    T = 900
+    x = synth.gen_x(77, T, dev)
+    sel = torch.full((T, 2), 9, dtype=torch.int64, device=dev)             # outside the window
+    sel[:820, 0] = 0                                                      # 820 picks: 4 blocks of 205
+    sel[800:840, 1] = 1
+    rw = (0.25 + 0.5 * torch.rand((T, 2), generator=torch.Generator().manual_seed(4))).half().to(dev)
+    pf = tier.PrefillBuffers(T, 2, 0, 2, 256, dev, bm=256, long=True).run(sel, rw)
+    assert pf.rbt[:int(pf.meta[1].item()), 2].tolist() == [205] * 4 + [40]
+    y = torch.zeros((T, 6144), dtype=torch.float32, device=dev)
+    moe4t.forward(x, pf.tok, pf.eid, pf.wt, pf.rbt, *lay.bank.tables(), *pf.scr, y, meta=pf.meta, npos=pf.F, nrb=pf.nrb_max,
+                  inv=pf.inv if ordered else None, topk=2)
+    parts = [moe_rows(lay, x, sel[:, k:k + 1], rw[:, k:k + 1], with_shared=False) for k in range(2)]
+    ref, lim = parts[0] + parts[1], bound(parts[0]) + bound(parts[1])      # (each pick's row has its own roundings)
+    none = ref.abs().amax(1) == 0
+    assert int(none.sum()) == 60 and not bool(y[none].any())
+    worst = ((y - ref).abs()[~none] / lim[~none]).max().item()
+    assert worst <= 1.0, worst
