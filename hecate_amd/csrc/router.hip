@@ -6,8 +6,8 @@
 //                    through LDS) and a select kernel (one wave per row); the kernel boundary replaces the reference's
 //                    last-block counter (exl3_router.py:74-83,130), whose cross-workgroup fences are costly on gfx950.
 //   large (R > 16) : an fp32 MFMA GEMM per (row tile, expert tile, segment) with the same chain order (one wave per tile up
-//                    to SR_ROWS rows, 128 rows x 64 experts per workgroup above), then a select kernel that folds the 8
-//                    segment sums and picks each row's top-k (one wave per row).
+//                    to 1536 rows of 256 experts, 128 rows x 64 experts per workgroup above), then a select kernel that
+//                    folds the 8 segment sums and picks each row's top-k (one wave per row).
 #include "hmoe_dev.h"
 
 namespace hmoe {
@@ -150,13 +150,13 @@ __global__ void __launch_bounds__(256) router_seg_mfma_kernel(
         }
 }
 
-// The same up to SR_ROWS rows, where the kernel above is a few workgroups of 24 serial chunks, a barrier each. One wave owns
-// 16 NR rows x 16 NE experts of one segment and needs no LDS and no barrier: lane l loads k 8(l/16) .. + 8 of row (expert) l % 16 of a chunk - 16 bytes of x, 32 of w - and a 4 x 4 transpose
-// between the four 16-lane groups (two permlane16 and two permlane32 swaps per four registers) gives each MFMA step its
-// operand, k 4 kk + l/16. The loads run D - 1 chunks ahead of their use.
-// What bounds it: the load latency of the 24 serial chunks. Router with its select, 256 experts, same bits: 33 rows 49.6 ->
-// 18.0 us, 150 rows 50.2 -> 26.1, 450 rows 53.8 -> 32.5.
-constexpr int SR_ROWS = 768;
+// The same for fewer rows, where the kernel above is a few workgroups of 24 serial chunks, a barrier each. One wave owns
+// 16 NR rows x 16 NE experts of one segment and needs no LDS and no barrier: lane l loads k 8(l/16) .. + 8 of row (expert)
+// l % 16 of a chunk - 16 bytes of x, 32 of w - and a 4 x 4 transpose between the four 16-lane groups (two permlane16 and two
+// permlane32 swaps per four registers) gives each MFMA step its operand, k 4 kk + l/16. The loads run D - 1 chunks ahead of
+// their use.
+// What bounds it: the load latency of the 24 serial chunks. Router with its select, 256 experts, same bits, the kernel above
+// against this one: 33 rows 49.6, 18.1 us; 150 rows 50.4, 26.1; 450 rows 53.3, 32.5.
 template <int NR, int NE>
 struct SegChunk { u32x4 x[NR]; f32x4 w[NE][2]; };
 
@@ -272,11 +272,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) r
         }
 }
 
+// launches it if that takes at most max_wg workgroups
 template <int NR, int NE>
-static void router_seg(const uint16_t* x, const float* wt, float* seg, int R, int K, int E, hipStream_t st)
+static bool router_seg(const uint16_t* x, const float* wt, float* seg, int R, int K, int E, int max_wg, hipStream_t st)
 {
-    const int ney = (E + 64 * NE - 1) / (64 * NE);
-    router_seg_wave_kernel<NR, NE><<<dim3((R + 16 * NR - 1) / (16 * NR) * ney, RSEG), 256, 0, st>>>(x, wt, seg, R, K, E, ney);
+    const int64_t nrt = (R + 16LL * NR - 1) / (16 * NR), ney = (E + 64 * NE - 1) / (64 * NE);
+    if (nrt * ney * RSEG > max_wg) return false;
+    router_seg_wave_kernel<NR, NE><<<dim3(nrt * ney, RSEG), 256, 0, st>>>(x, wt, seg, R, K, E, ney);
+    return true;
 }
 
 // large path, 2: fold the segments in order, select; one wave per row; optional f16 copy of x
@@ -311,7 +314,11 @@ __global__ void __launch_bounds__(256) router_select_kernel(const float* __restr
             const u32x4 v = *(const u32x4*) (x + (size_t) r * K + k);
             f16x8 o;
             #pragma unroll
-            for (int q = 0; q < 4; ++q) { o[2 * q] = (_Float16) __uint_as_float(v[q] << 16); o[2 * q + 1] = (_Float16) __uint_as_float(v[q] & 0xffff0000u); }
+            for (int q = 0; q < 4; ++q)
+            {
+                o[2 * q] = (_Float16) __uint_as_float(v[q] << 16);
+                o[2 * q + 1] = (_Float16) __uint_as_float(v[q] & 0xffff0000u);
+            }
             *(f16x8*) (xh + (size_t) r * K + k) = o;
         }
 }
@@ -355,15 +362,18 @@ extern "C" int hmoe_router_fused(const void* x, const float* wt, const float* bi
         if (int rc = HMOE_LAUNCHED("router_fused")) return rc;
         return router_select_small(logits, bias, R, E, topk, scale, sel, rw, st);
     }
-    // Small tiles while the launch would not fill the chip otherwise (measured with the select, us: 64 rows 18.1 with 16 x 16
-    // per wave, 24.3 with 16 x 32; 150 rows 27.5, 26.1 and 30.5 with 32 x 32; 450 rows 47.7, 41.7, 32.5). From ~700 rows the
-    // LDS-staged tiles reuse their operands more (700 rows 54.5 against 52.1, 1000 rows 54.7 against 53.5, 2048 rows 83
-    // against 95; 64 x 32 per wave 1000 rows 49.6, 1300 rows 84.9 against 79.1, 8192 rows 320 against 282).
+    // The smallest wave tiles whose launch is one workgroup a CU: a wave then has least to do in each of its serial chunks,
+    // and a second workgroup on a CU costs more than a larger tile. Tiles of 32 x 32 up to three workgroups a CU; past that
+    // the LDS-staged kernel, which reads its operands once for more rows. Router with its select, 256 experts, us, tiles of
+    // 16 x 16, 16 x 32 and 32 x 32 a wave and the LDS-staged kernel:
+    //   128 rows 18.8, 25.8, 31.1, -        129 rows 27.6, 25.4, 30.6, -       256 rows 28.8, 26.4, 31.4, -
+    //   257 rows 38.0, 41.0, 31.5, -        512 rows 47.3, 42.0, 32.6, 51.9    1024 rows 84.0, 72.6, 53.6, 54.6
+    //   1025 rows 92.3, 86.6, 72.4, 78.4    1536 rows 120, 103, 75.3, 79.5     1537 rows 129, 117, 91.0, 80.2
+    // and 128 experts: 256 rows 18.7, 25.9, 31.4, -, 500 rows 30.3, 26.9, 31.6, 52.1, 3000 rows 123, 107, 78.4, 83.0
+    constexpr int CUS = 256;
     const uint16_t* xb = (const uint16_t*) x;
-    if (R <= 96) router_seg<1, 1>(xb, wt, logits, R, K, E, st);
-    else if (R <= 320) router_seg<1, 2>(xb, wt, logits, R, K, E, st);
-    else if (R <= SR_ROWS) router_seg<2, 2>(xb, wt, logits, R, K, E, st);
-    else
+    if (!router_seg<1, 1>(xb, wt, logits, R, K, E, CUS, st) && !router_seg<1, 2>(xb, wt, logits, R, K, E, CUS, st) &&
+        !router_seg<2, 2>(xb, wt, logits, R, K, E, 3 * CUS, st))
         router_seg_mfma_kernel<<<dim3((R + SM_R - 1) / SM_R, (E + SM_E - 1) / SM_E, RSEG), 256, 0, st>>>(xb, wt, logits, R, K,
                                                                                                        E);
     router_select_kernel<<<(R + 3) / 4, 256, 0, st>>>(logits, bias, R, E, topk, scale, sel, rw, (const uint16_t*) x,

@@ -12,7 +12,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("R,E,K,adv", [
     (17, 256, 6144, False), (32, 250, 6144, True), (33, 9, 6144, False), (96, 256, 6144, False), (97, 130, 6144, True),
     (320, 256, 6144, False), (321, 33, 6144, False), (768, 256, 6144, False), (769, 256, 6144, False),
-    (50, 256, 256, True), (200, 70, 512, False), (400, 256, 1280, False)])
+    (50, 256, 256, True), (200, 70, 512, False), (400, 256, 1280, False),
+    (128, 256, 512, True), (129, 256, 512, False), (256, 256, 512, False), (257, 250, 512, True), (512, 64, 512, False),
+    (513, 64, 512, True), (500, 128, 512, False), (1536, 256, 512, False), (1537, 256, 512, True), (1536, 129, 512, False)])
 def test_router_tiles(R, E, K, adv):
     from hecate_amd import router
     from test_gpu_parity import _adversarial, u16
