@@ -17,13 +17,15 @@
 // one wait placed by hand is a wave's own stage loads before the barrier that publishes them; the loads after a stage in
 // program order are fixed (sched_barrier around each bundle), so that count is a compile-time constant too.
 //
-// Measured on one layer of 256 experts (gate/up + down launch, against the same tiles with two 128-k stages and a 2-deep
-// weight ring whose waits also waited for the stage loads; bits equal): 33 tokens 413 + 212 -> 343 + 184 us (160 experts,
-// 6.0 and 5.6 TB/s of weights), 150 tokens 634 + 327 -> 540 + 290, 450: 677 + 351 -> 582 + 320, 2048: 1011 + 556 -> 961 +
-// 537. At 33 to ~500 tokens the weight stream bounds it (a read-only stream reaches 6.05 TB/s); at 2048 the issue slots: a
-// fragment costs 13 VALU instructions of dequantisation and NT MFMAs at ~5 issue cycles each, against 16 per MFMA in
-// the matrix core, at a clock the power limit holds at 1.6-1.9 GHz. An epilogue chosen at run time instead of by template
-// spills registers in the k loop (+5 to 8 %).
+// Measured on one layer of 256 experts, the shared expert included, whole moe4p.forward calls against the same tiles with
+// two 128-k stages, a 2-deep weight ring whose waits also waited for the stage loads, and the shared expert in launches of
+// its own (bits equal): 33 tokens 688 -> 565 us, 150 tokens 1046 -> 871, 450 1145 -> 975, 1000 1366 -> 1232, 2048 1786 ->
+// 1736. At 33 to ~500 tokens the weight stream bounds it (33 tokens, without the shared expert: 3.1 GB of 165 experts in 528
+// us, 5.9 TB/s; a read-only stream reaches 6.05). At 2048 the issue slots (counters of the gate/up launch, per SIMD): 976 K
+// cycles of MFMA and 700 K of other VALU, mostly the 13 instructions a fragment costs to dequantise, in a launch of 1930 K,
+// at a clock the power limit holds at 1.6-1.9 GHz; waits on loads are 0.14 of the wave cycles, waits to issue 0.52. At 1000
+// tokens of uneven popularity neither is full: 531 K and 592 K of 1496 K cycles, and 4.3 TB/s. An epilogue chosen at run
+// time instead of by template spills registers in the k loop (+5 to 8 %).
 #pragma once
 #include "hmoe_dev.h"
 
