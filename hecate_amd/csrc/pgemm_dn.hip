@@ -10,14 +10,16 @@ int hmoe::grouped_down(const PgArgs& a, int epi, hipStream_t st)
     // life is its prologue (256 experts: 150 tokens 843 with one, 823 with three; 1000 tokens 1128, 1108). One where that
     // leaves CUs without a workgroup, which then run three times as long: tables of few experts (8 experts: 450 tokens 71
     // with one, 94 with three; 2048 tokens 116, 154; 48 experts: 187, 192 and 325, 332; from 64 on three again: 244, 237 and
-    // 415, 414), or few picks (17 tokens: 96 experts 159, 167; 256 experts 365, 364). Beside the shared expert's blocks the
+    // 415, 414), or few picks (17 tokens: 96 experts 159, 167; 256 experts 365, 364). Not where the plan has room for many
+    // short blocks of them (32 experts, 2048 tokens in blocks of 16, 32 and 64 picks: 3623 with one, 3440 with three; 2212,
+    // 2134; 1591, 1564; the room is 32 + picks / block, 160 in blocks of 128: 1193, 1199). Beside the shared expert's blocks the
     // routed ones spread over fewer free slots, and the line is higher (33 tokens: 64 experts 226, 241; 450: 279, 293 and 96
     // experts 400, 409; 128 experts 520, 518).
     // Shared: one, its serial chain over k being the launch's length beside few experts (33 tokens, 8 experts 145 with one,
     // 204 with three; 450 tokens, 32 experts 230, 290; 1000 tokens, 256 experts 1224, 1223). (The kernel takes the count at
     // run time: with a constant one it spills two registers.)
     PgArgs g = a;
-    g.ncb = a.np < 200 || a.n_tab < (a.sh0 ? 128 : 64) ? 1 : 3;
+    g.ncb = a.np < 200 || (a.n_tab < (a.sh0 ? 128 : 64) && a.nrb < 288) ? 1 : 3;
     g.shb = 1;
     pg_shared_blocks(g);
     const dim3 grid = pgemm_grid(a.nrb, H / 256 / g.ncb, g.nsh * g.ncb / g.shb);
