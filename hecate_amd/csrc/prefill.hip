@@ -6,7 +6,7 @@
 // GEMMs: workgroup = (row block of picks of one expert, 128 gate/up or 256 down output columns); see pgemm.h, and
 // pgemm16_kernel for long chunks of many picks an expert. gu fuses act = silu(g) * u * w (f16), down writes d = W_d act as
 // f16 rows, whose picks fin sums per token in top-k order in fp32 (or, when no inverse map is given, down adds its fp32 sums
-// into out with atomics, as p4_fin_kernel). The shared expert's projections ride in the same launches (moe4p up to 4096
+// into out with atomics, as p4_fin_kernel). The shared expert's projections ride in the same launches (moe4p up to 3584
 // tokens) or run on the dense MFMA GEMMs of shared_gemm.hip.
 #include "pgemm.h"
 
@@ -665,11 +665,12 @@ static int moe4p_run(const void* x, const int* tok, const float* wt, const int* 
     // gate/up, then down into d rows for the ordered combine (inv given) or added into out[tok] by its epilogue (no
     // inverse map: the atomic combine of p4_fin_kernel)
     // The shared expert (every token) rides in the same two launches: act rows ps.. = f16(silu(gate x) up x), then down
-    // into d rows ps.. (f16), which the ordered combine adds after each token's picks. Past 4096 tokens it takes the
-    // dense launches instead, whose larger tiles are the faster once there are enough of them (us, riding against apart:
-    // 8192 tokens, 8 experts 1040, 959, 256 experts 5711, 5616; 6000 tokens 750, 701 and 4303, 4246; 4096 tokens 562, 558 and
-    // 3126, 3193; 3000 tokens, 8 experts 381, 458).
-    const bool sh = sh_gw != nullptr, apart = sh && T > 4096;
+    // into d rows ps.. (f16), which the ordered combine adds after each token's picks. Past 3584 tokens it takes the
+    // dense launches instead, whose larger tiles are the faster once there are enough of them (us, riding against apart, 8,
+    // 32 and 256 experts: 3072 tokens 403, 415; 555, 548; 2198, 2191; 3584 tokens 485, 469; 664, 673; 2529, 2506; 3840 tokens
+    // 533, 493; 733, 696; 2743, 2708; 4096 tokens 559, 504; 813, 758; 3101, 3044; 8192 tokens, 8 and 256: 1040, 959; 5711,
+    // 5616).
+    const bool sh = sh_gw != nullptr, apart = sh && T > 3584;
     PgArgs g{};
     g.xin = (const _Float16*) xb; g.tok = tok; g.wt = wt; g.rbt = rbt; g.meta = meta;
     g.w0 = gw; g.w1 = uw; g.s0 = gs; g.s1 = us; g.out = a;

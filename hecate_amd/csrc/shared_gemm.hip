@@ -1,5 +1,5 @@
 // shared_gemm.hip - the shared expert over a chunk by itself (hmoe_shared_forward, hmoe_shared_rows, and moe4p's calls of
-// more than 4096 tokens) as hand-written dense MFMA GEMMs (f16 operands, fp32 accumulation); in shorter moe4p calls it
+// more than 3584 tokens) as hand-written dense MFMA GEMMs (f16 operands, fp32 accumulation); in shorter moe4p calls it
 // rides in the grouped GEMM's launches (pgemm.h). The shared expert is a dense bf16 MLP (its weights are exact in f16), run over
 // every token of the chunk; the reference keeps it outside its routed op at prefill (runtime/tier/tier_split.py:548-560,
 // the model's own shared-expert forward). gate and up run as one GEMM whose epilogue writes act = f16(silu(g) u); down

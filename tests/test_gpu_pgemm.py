@@ -92,22 +92,22 @@ def test_wide_tables(lay, n):
 
 
 def test_shared_apart(lay):
-    """past 4096 tokens the shared expert runs in launches of its own: its rows of the first 4096 tokens against the ones of
+    """past 3584 tokens the shared expert runs in launches of its own: its rows of the first 3584 tokens against the ones of
     the grouped launches, the same sums in the same order, so the same bits"""
     from hecate_amd import moe4p, synth, tier
     dev = lay.device
-    x = synth.gen_x(61, 4099, dev)
-    sel = torch.full((4099, 1), 2, dtype=torch.int64, device=dev)         # outside the window, but for a few tokens
+    x = synth.gen_x(61, 3587, dev)
+    sel = torch.full((3587, 1), 2, dtype=torch.int64, device=dev)         # outside the window, but for a few tokens
     sel[::9] = 0
-    rw = torch.full((4099, 1), 0.5, dtype=torch.float16, device=dev)
+    rw = torch.full((3587, 1), 0.5, dtype=torch.float16, device=dev)
     ys = []
-    for T in (4096, 4099):
+    for T in (3584, 3587):
         pf = tier.PrefillBuffers(T, 1, 0, 2, 256, dev).run(sel[:T], rw[:T])
         y = torch.zeros((T, 6144), dtype=torch.float32, device=dev)
         moe4p.forward(x[:T], pf.tok, pf.eid, pf.wt, pf.rbt, *lay.bank.tables(), *pf.scr, y, inv=pf.inv, meta=pf.meta, topk=1,
                       npos=T, nrb=pf.nrb_max, shared=lay.shared_rows())
         ys.append(y)
-    assert bool(ys[1].abs().amax(1).all()) and torch.equal(ys[0].view(torch.int32), ys[1][:4096].view(torch.int32))
+    assert bool(ys[1].abs().amax(1).all()) and torch.equal(ys[0].view(torch.int32), ys[1][:3584].view(torch.int32))
 
 
 @pytest.mark.parametrize("ordered", (True, False))
