@@ -505,7 +505,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     {
         // the shared expert's blocks come first: they are the longest, and the rest fills in around them. The token blocks of
         // one column block go to consecutive workgroups of one XCD, which then reads its weights once (NCB / shb is a
-        // multiple of 8: 16 in gate/up, 24 or 8 in down).
+        // multiple of 8: 16 in gate/up, 24 or 8 in down, where shb divides ncb).
         const int ns = a.nsh * (NCB / a.shb);
         if (i < ns)
         {

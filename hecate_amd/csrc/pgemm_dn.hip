@@ -16,11 +16,12 @@ int hmoe::grouped_down(const PgArgs& a, int epi, hipStream_t st)
     // routed ones spread over fewer free slots, and the line is higher (33 tokens: 64 experts 226, 241; 450: 279, 293 and 96
     // experts 400, 409; 128 experts 520, 518).
     // Shared: one, its serial chain over k being the launch's length beside few experts (33 tokens, 8 experts 145 with one,
-    // 204 with three; 450 tokens, 32 experts 230, 290; 1000 tokens, 256 experts 1224, 1223). (The kernel takes the count at
-    // run time: with a constant one it spills two registers.)
+    // 204 with three; 450 tokens, 32 experts 230, 290; 256 experts, 64 tokens 732, 748). Three in longer chunks beside nearly
+    // all experts, where the routed part is several times the chain and the prologues count (256 experts: 150 tokens 875,
+    // 875; 300 917, 915; 1000 1223, 1218, uneven 1216, 1208; 2048 1724, 1722; but 176 experts, 2048 tokens 1230, 1238).
     PgArgs g = a;
     g.ncb = a.np < 200 || (a.n_tab < (a.sh0 ? 128 : 64) && a.nrb < 288) ? 1 : 3;
-    g.shb = 1;
+    g.shb = g.ncb == 3 && a.n_tab >= 192 && a.T > 256 ? 3 : 1;
     pg_shared_blocks(g);
     const dim3 grid = pgemm_grid(a.nrb, H / 256 / g.ncb, g.nsh * g.ncb / g.shb);
     if (grid.x == 0) return HMOE_OK;

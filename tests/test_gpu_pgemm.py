@@ -71,8 +71,9 @@ def test_shared_blocks(lay, T):
 
 @pytest.mark.parametrize("n", NS)
 def test_wide_tables(lay, n):
-    """the down launch with three column blocks a workgroup (tables of 128 experts, 200 picks or more of room) against the
-    one of few experts: the same sums in the same order, so the same bits, the shared expert's rows among them"""
+    """the down launch with three column blocks a workgroup (tables of 128 experts, 200 picks or more of room; from 257 tokens
+    and 192 experts the shared expert's blocks too) against the one of few experts: the same sums in the same order, so the
+    same bits, the shared expert's rows among them"""
     from hecate_amd import moe4p, synth, tier
     dev = lay.device
     T = n + 3
@@ -82,13 +83,14 @@ def test_wide_tables(lay, n):
     rw = torch.full((T, 1), 0.5, dtype=torch.float16, device=dev)
     for shared in (None, lay.shared_rows()):
         ys = []
-        for room, experts in ((T, 2), (max(T, 200), 128)):
+        for room, experts in ((T, 2), (max(T, 200), 128), (max(T, 200), 192)):
             pf = tier.PrefillBuffers(room, 1, 0, experts, 256, dev).run(sel, rw)
             y = torch.zeros((T, 6144), dtype=torch.float32, device=dev)
             moe4p.forward(x, pf.tok, pf.eid, pf.wt, pf.rbt, *[t.repeat(experts // 2) for t in lay.bank.tables()], *pf.scr, y,
                           inv=pf.inv[:T], meta=pf.meta, topk=1, npos=pf.F, nrb=pf.nrb_max, shared=shared)
             ys.append(y)
-        assert bool(ys[0].any()) and torch.equal(ys[0].view(torch.int32), ys[1].view(torch.int32)), (n, shared is None)
+        for y in ys[1:]:
+            assert bool(y.any()) and torch.equal(ys[0].view(torch.int32), y.view(torch.int32)), (n, shared is None)
 
 
 def test_shared_apart(lay):
